@@ -1,0 +1,302 @@
+"""The workloads this library's speed is measured on.
+
+Each case is one pass through a public entry point as a planning program calls
+it: edge validation on device buffers (roadmap and tree edges), pose checks on
+host buffers (start and goal sampling), nearest-node search on device trees,
+single solves, batched solves and a served burst of requests.  Sizes and
+settings are those of the benchmark, the tests and the serving load generator.
+
+    listed()            the cases
+    draw(rng)           one more case of the same ranges
+    prepare(case, seed) inputs and handles of one pass, from the seed alone
+    run(state)          the pass
+    exact(case, seed)   the computed numbers in 64 bits, where there are some
+    work(case)          bytes and flops a pass cannot do without
+    tolerance(case)     how far another correct implementation may be off
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+import prrtc_amd as P
+from prrtc_amd import lib, loadgen, workloads
+from prrtc_amd import scenes as S
+from prrtc_amd.autotune import SETTINGS as CLASS_SETTINGS
+from prrtc_amd.robots import DOF, fixed_spheres, limits
+
+# FK multiply-adds of one pose (the reference's generated code, counted by
+# prrtc_amd.accounting; UR5 by the same rule from its table)
+FK_FLOPS = {"panda": 1079, "fetch": 962, "baxter": 1750, "ur5": 600}
+# queries a wavefront group shares (the library's own default)
+NEAREST_WAVES = 4
+# rows a plan may have (the longest plan of the test suite has 251)
+PATH_ROWS = 512
+
+
+# ------------------------------------------------------------------- cases
+
+def listed():
+    return [
+        # the neighbours of one new roadmap node: the smallest call, a launch
+        {"name": "edges_panda_query", "kind": "edges", "robot": "panda", "scene": "cuboids", "n": 64, "g": 32,
+         "local": True, "max_len": 1.0, "free": 0.6},
+        # a batch of roadmap edges between free configurations, most of them
+        # free, a ragged count
+        {"name": "edges_fetch_roadmap", "kind": "edges", "robot": "fetch", "scene": "mixed", "n": 10_007, "g": 64,
+         "local": True, "max_len": 0.5, "free": 0.6},
+        # uniform edges of a 14-joint robot in a shelf, short interpolation
+        {"name": "edges_baxter_uniform", "kind": "edges", "robot": "baxter", "scene": "shelf", "n": 30_011, "g": 32,
+         "local": False, "max_len": 0.5, "free": 0.1},
+        # the edge microbenchmark: 1M uniform edges, 24 cuboids and 8 cylinders
+        {"name": "edges_panda_bulk", "kind": "edges", "robot": "panda", "scene": "cuboids", "n": 1_000_000, "g": 128,
+         "local": False, "max_len": 0.5, "free": 0.07},
+        # start/goal sampling: a block of uniform poses checked from the host
+        {"name": "poses_fetch", "kind": "poses", "robot": "fetch", "scene": "mixed", "n": 4096},
+        # one query of one mid-sized tree: latency
+        {"name": "nearest_one", "kind": "nearest", "dof": 14, "nodes": 20_011, "trees": 1, "queries": 1},
+        # one query of each of many large trees: every byte from memory once
+        {"name": "nearest_stream", "kind": "nearest", "dof": 8, "nodes": 100_000, "trees": 256, "queries": 1},
+        # a round of queries per tree (one per new configuration)
+        {"name": "nearest_round", "kind": "nearest", "dof": 7, "nodes": 50_000, "trees": 64, "queries": 64},
+        # one problem among spheres, as a program that plans once calls it
+        {"name": "solve_panda", "kind": "solve", "robot": "panda", "scene": "spheres", "problems": 1, "nnc": 128,
+         "g": 32, "max_iters": 2000},
+        # several cluttered problems, one call each
+        {"name": "solve_fetch_seq", "kind": "solve", "robot": "fetch", "scene": "mixed", "problems": 8, "nnc": 256,
+         "g": 64, "max_iters": 500},
+        # an uneven mix of robots in shelves, one call
+        {"name": "batch_mix", "kind": "batch", "baxter": 32, "panda": 64, "fetch": 32, "nnc": 64, "g": 128,
+         "max_iters": 1000},
+        # a burst of requests of all robots through the server
+        {"name": "serve_burst", "kind": "serve", "requests": 32, "nnc": 64, "g": 64, "max_iters": 600},
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["edges", "edges", "edges", "nearest", "nearest", "poses", "solve", "batch", "serve"])
+    robot = rng.choice(["panda", "fetch", "baxter", "ur5"])
+    scene = rng.choice(["spheres", "mixed", "shelf", "cuboids"])
+    if kind == "edges":
+        g = rng.choice([16, 32, 50, 64, 100, 128])
+        local = rng.random() < 0.5
+        # local edges have free ends, found by rejection: a bounded count
+        n = _log_int(rng, 48, 30_000 if local else 300_000)
+        return {"kind": kind, "robot": robot, "scene": scene, "n": n, "g": g, "local": local,
+                "max_len": rng.choice([0.5, 1.0]), "free": 0.6 if local else 0.1}
+    if kind == "poses":
+        return {"kind": kind, "robot": robot, "scene": scene, "n": _log_int(rng, 64, 65_536)}
+    if kind == "nearest":
+        nodes = _log_int(rng, 1, 100_000)
+        trees = _log_int(rng, 1, 256)
+        return {"kind": kind, "dof": rng.choice([3, 7, 8, 14]), "nodes": nodes, "trees": trees,
+                "queries": min(_log_int(rng, 1, 128), max(1, 8192 // trees))}
+    nnc = rng.choice([32, 64, 100, 128, 256, 512])
+    g = rng.choice([32, 64, 100, 128])
+    if kind == "solve":
+        return {"kind": kind, "robot": robot, "scene": scene, "problems": rng.randint(1, 4), "nnc": nnc, "g": g,
+                "max_iters": rng.choice([50, 100, 300])}
+    if kind == "batch":
+        return {"kind": kind, "baxter": rng.randint(0, 16), "panda": rng.randint(1, 32), "fetch": rng.randint(0, 16),
+                "nnc": rng.choice([32, 64, 128]), "g": g, "max_iters": rng.choice([100, 300, 500])}
+    return {"kind": kind, "requests": rng.randint(1, 32), "nnc": rng.choice([32, 64, 128]), "g": g,
+            "max_iters": rng.choice([100, 300, 600])}
+
+
+# ------------------------------------------------------------------ inputs
+
+def _scene(robot, kind, seed):
+    avoid = fixed_spheres(robot)
+    make = {
+        "spheres": lambda s: S.scene_spheres(s, 12, avoid=avoid),
+        "mixed": lambda s: S.scene_mixed(s, 8, 64, avoid=avoid),
+        "shelf": lambda s: S.scene_shelf(s, 4, 128, avoid=avoid),
+        "cuboids": lambda s: S.scene_obb_cylinders(s, 24, 8, avoid=avoid),
+    }[kind]
+    return workloads.feasible_scene(robot, make, seed, np.random.default_rng(seed), min_free=0.02)
+
+
+def _poses(robot, n, gen):
+    lo, span = (torch.from_numpy(v).cuda() for v in limits(robot))
+    return lo + span * torch.rand((n, DOF[robot]), generator=gen, device="cuda")
+
+
+def _edges(robot, scene, n, max_len, local, gen):
+    """n edges (a, b), |b - a| ~ U(0, max_len] in a uniform direction, both
+    ends in the joint limits; `local`: both ends collision-free."""
+    lo, span = (torch.from_numpy(v).cuda() for v in limits(robot))
+    hi = lo + span
+    got, have = [], 0
+    while have < n:
+        m = max(4096, 2 * (n - have))
+        a = _poses(robot, m, gen)
+        u = torch.randn(a.shape, generator=gen, device="cuda")
+        u /= u.norm(dim=1, keepdim=True)
+        b = a + max_len * (1.0 - torch.rand((m, 1), generator=gen, device="cuda")) * u
+        ok = ((b >= lo) & (b <= hi)).all(1)
+        e = torch.stack([a, b], 1)[ok]
+        if local:
+            ends = P.check_poses(robot, scene, e.reshape(-1, e.shape[-1]).cpu().numpy()).reshape(-1, 2)
+            e = e[torch.from_numpy(ends.all(1)).cuda()]
+        got.append(e)
+        have += len(e)
+    return torch.cat(got)[:n].contiguous()
+
+
+def _problems(case, seed):
+    robot, n, kind = case["robot"], case["problems"], case["scene"]
+    out = []
+    for i in range(n):
+        s = seed + 1009 * i
+        sc = _scene(robot, kind, s)
+        q = workloads.free_poses(robot, sc, 2, np.random.default_rng(s))
+        out.append({"robot": robot, "start": q[0], "goals": q[1][None], "scene": sc})
+    return out
+
+
+def _settings(case, robot, seed):
+    """The robot class's planner settings at the case's size."""
+    return dict(CLASS_SETTINGS[robot], num_new_configs=case["nnc"], granularity=case["g"],
+                max_iters=case["max_iters"], max_samples=50_000, seed=1 + seed % 1000)
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    if kind == "edges":
+        scene = _scene(case["robot"], case["scene"], seed)
+        edges = _edges(case["robot"], scene, case["n"], case["max_len"], case["local"], gen)
+        return {"case": case, "scene": torch.from_numpy(P.pack_scene(scene)).cuda(), "edges": edges,
+                "free": torch.zeros(case["n"], dtype=torch.uint8, device="cuda")}
+    if kind == "poses":
+        scene = _scene(case["robot"], case["scene"], seed)
+        return {"case": case, "scene": scene, "poses": _poses(case["robot"], case["n"], gen).cpu().numpy()}
+    if kind == "nearest":
+        trees, queries, cap = _trees(case, gen)
+        nq = case["trees"] * case["queries"]
+        return {"case": case, "trees": trees, "queries": queries, "cap": cap,
+                "idx": torch.zeros(nq, dtype=torch.int32, device="cuda"),
+                "dist2": torch.zeros(nq, dtype=torch.float32, device="cuda")}
+    if kind == "solve":
+        st = _settings(case, case["robot"], seed)
+        return _with_paths({"case": case, "problems": _problems(case, seed), "settings": st})
+    if kind == "batch":
+        probs = workloads.c3_problems(case["baxter"], case["panda"], case["fetch"], seed=seed)
+        st = [_settings(case, p["robot"], seed) for p in probs]
+        return _with_paths({"case": case, "problems": probs, "settings": st})
+    pool = loadgen.request_pool(case["requests"], seed=seed)
+    st = dict(loadgen.SERVE_SETTINGS, num_new_configs=case["nnc"], granularity=case["g"],
+              max_iters=case["max_iters"], seed=1 + seed % 1000)
+    return _with_paths({"case": case, "problems": pool, "settings": st, "server": P.Server(path_cap=PATH_ROWS)})
+
+
+def _with_paths(state):
+    state["paths"] = np.zeros((len(state["problems"]), PATH_ROWS, lib.MAX_DOF), dtype=np.float32)
+    return state
+
+
+def _trees(case, gen):
+    # nodes and queries uniform in a joint range of 2 pi, SoA per tree
+    cap = (case["nodes"] + 1023) // 1024 * 1024
+    trees = (torch.rand((case["trees"], case["dof"], cap), generator=gen, device="cuda") - 0.5) * (2 * math.pi)
+    queries = (torch.rand((case["trees"], case["queries"], case["dof"]), generator=gen, device="cuda") - 0.5) * (
+        2 * math.pi)
+    return trees, queries, cap
+
+
+# -------------------------------------------------------------------- pass
+
+def _plans(state, outs):
+    """The plans of a pass: everything but the times and the lane count, which
+    depends on the launch shape.  Paths lie in rows of the state's buffer."""
+    for i, (_, path) in enumerate(outs):
+        state["paths"][i, :path.shape[0], :path.shape[1]] = path
+    return {"paths": state["paths"],
+            "numbers": np.array([[r["solved"], r["status"], r["iters"], r["start_tree_size"], r["goal_tree_size"],
+                                  r["path_length"], r["path_nodes"], r["edge_checks"]] for r, _ in outs]),
+            "cost": np.array([r["cost"] for r, _ in outs], dtype=np.float32)}
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "edges":
+        P.validate_edges_async(case["robot"], state["scene"].data_ptr(), state["scene"].numel(),
+                               state["edges"].data_ptr(), case["n"], case["g"], state["free"].data_ptr(),
+                               torch.cuda.current_stream().cuda_stream)
+        return state["free"]
+    if kind == "poses":
+        return P.check_poses(case["robot"], state["scene"], state["poses"])
+    if kind == "nearest":
+        P.nearest_async(case["dof"], state["trees"].data_ptr(), state["cap"], case["nodes"], case["trees"],
+                        state["queries"].data_ptr(), case["queries"], NEAREST_WAVES, state["idx"].data_ptr(),
+                        state["dist2"].data_ptr(), torch.cuda.current_stream().cuda_stream)
+        return {"idx": state["idx"], "dist2": state["dist2"]}
+    if kind == "solve":
+        return _plans(state, [P.solve(p["robot"], p["start"], p["goals"], p["scene"], state["settings"],
+                                      path_cap=PATH_ROWS) for p in state["problems"]])
+    if kind == "batch":
+        results, paths, _ = P.solve_batch(state["problems"], state["settings"], path_cap=PATH_ROWS)
+        return _plans(state, list(zip(results, paths)))
+    srv = state["server"]
+    tickets = [srv.submit(p, state["settings"]) for p in state["problems"]]
+    return _plans(state, [srv.poll(t)[:2] for t in tickets])
+
+
+# -------------------------------------------------------------- references
+
+def exact(case, seed):
+    """Squared distances in 64 bits; verdicts are bytes and a plan follows
+    from thousands of verdicts, so neither has a computed number to compare."""
+    if case["kind"] != "nearest":
+        return None
+    trees, queries, _ = _trees(case, torch.Generator(device="cuda").manual_seed(seed))
+    n = case["nodes"]
+    out = []
+    for t in range(case["trees"]):
+        x, q = trees[t, :, :n].double(), queries[t].double()
+        for j in range(case["queries"]):
+            out.append(((x - q[j][:, None]) ** 2).sum(0).min())
+    return {"idx": None, "dist2": torch.stack(out)}
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "edges":
+        # a free edge needs every pose's kinematics, a colliding one a pose's
+        poses = case["n"] * (case["free"] * case["g"] + 1.0 - case["free"])
+        return {"bytes": case["n"] * (8 * DOF[case["robot"]] + 1), "flops": poses * FK_FLOPS[case["robot"]]}
+    if kind == "poses":
+        return {"bytes": case["n"] * (4 * DOF[case["robot"]] + 1), "flops": case["n"] * FK_FLOPS[case["robot"]]}
+    if kind == "nearest":
+        per_tree = 4 * case["dof"] * case["nodes"]
+        queries = case["trees"] * case["queries"]
+        return {"bytes": case["trees"] * per_tree + queries * (4 * case["dof"] + 8),
+                "flops": 3 * case["dof"] * case["nodes"] * queries}
+    # one round of every problem: each slot samples, searches the tree and
+    # validates an edge of g poses
+    if kind == "batch":
+        robots = [("baxter", case["baxter"]), ("panda", case["panda"]), ("fetch", case["fetch"])]
+    elif kind == "solve":
+        robots = [(case["robot"], case["problems"])]
+    else:
+        robots = [("panda", case["requests"])]
+    poses = sum(n * FK_FLOPS[r] for r, n in robots) * case["nnc"] * case["g"]
+    return {"bytes": sum(n * 4 * DOF[r] for r, n in robots) * case["nnc"], "flops": poses}
+
+
+def tolerance(case):
+    # The library states its rounding (one fmaf chain per distance, ties to
+    # the smaller index; every verdict an explicit chain of fmaf) and that a
+    # plan is the same alone, batched and served, whatever the launch shape:
+    # verdict bytes, plan numbers and paths are the same bit for bit.
+    if case["kind"] == "nearest":
+        # a distance summed in another order (one query: 1.4e-7 from 64 bits)
+        return {"rel": 5e-7, "max": 1e-6, "differ": 1e-4}
+    return "exact"
