@@ -42,17 +42,17 @@ def listed():
     return [
         # the neighbours of one new roadmap node: the smallest call, a launch
         {"name": "edges_panda_query", "kind": "edges", "robot": "panda", "scene": "cuboids", "n": 64, "g": 32,
-         "local": True, "max_len": 1.0, "free": 0.6},
+         "local": True, "max_len": 1.0, "free": 0.9},
         # a batch of roadmap edges between free configurations, most of them
         # free, a ragged count
         {"name": "edges_fetch_roadmap", "kind": "edges", "robot": "fetch", "scene": "mixed", "n": 10_007, "g": 64,
-         "local": True, "max_len": 0.5, "free": 0.6},
+         "local": True, "max_len": 0.5, "free": 0.95},
         # uniform edges of a 14-joint robot in a shelf, short interpolation
         {"name": "edges_baxter_uniform", "kind": "edges", "robot": "baxter", "scene": "shelf", "n": 30_011, "g": 32,
-         "local": False, "max_len": 0.5, "free": 0.1},
+         "local": False, "max_len": 0.5, "free": 0.25},
         # the edge microbenchmark: 1M uniform edges, 24 cuboids and 8 cylinders
         {"name": "edges_panda_bulk", "kind": "edges", "robot": "panda", "scene": "cuboids", "n": 1_000_000, "g": 128,
-         "local": False, "max_len": 0.5, "free": 0.07},
+         "local": False, "max_len": 0.5, "free": 0.15},
         # start/goal sampling: a block of uniform poses checked from the host
         {"name": "poses_fetch", "kind": "poses", "robot": "fetch", "scene": "mixed", "n": 4096},
         # one query of one mid-sized tree: latency
@@ -89,7 +89,7 @@ def draw(rng):
         # local edges have free ends, found by rejection: a bounded count
         n = _log_int(rng, 48, 30_000 if local else 300_000)
         return {"kind": kind, "robot": robot, "scene": scene, "n": n, "g": g, "local": local,
-                "max_len": rng.choice([0.5, 1.0]), "free": 0.6 if local else 0.1}
+                "max_len": rng.choice([0.5, 1.0]), "free": 0.95 if local else 0.2}
     if kind == "poses":
         return {"kind": kind, "robot": robot, "scene": scene, "n": _log_int(rng, 64, 65_536)}
     if kind == "nearest":
