@@ -260,7 +260,7 @@ def main():
         "roofline": {"bound": "valu", "achieved": achieved / 1e12, "peak": PEAK_FP32_PACKED / 1e12,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_PACKED,
                      "frac_of_nonpacked_peak": achieved / PEAK_FP32, "traffic": traffic,
-                     "kernel": "k_validate_edges<PandaRobot, true>", "kernel_ms": roof_ms,
+                     "kernel": "k_validate_edges<PandaRobot>", "kernel_ms": roof_ms,
                      "flops_per_pose": per_pose, "poses_per_launch": n_roof * g, "valu_counters": valu},
     }
     paths_to_check = []   # (robot, scene, path, g)

@@ -41,9 +41,12 @@ __host__ __device__ inline int scene_payload_f4(int n_sph, int n_cap, int n_zcap
 }
 
 // Obstacle tables as seen by one workgroup: counts in registers (uniform),
-// payload behind a pointer (LDS after staging, or global).
+// payload in LDS (staged).  `ball` holds a bounding ball (centre, padded
+// radius) of every obstacle that is not a sphere, in table order (capsules,
+// z-capsules, cuboids, z-cuboids); a sphere's row is its own ball.  An
+// obstacle is named by its index in the whole scene, spheres first.
 struct Obstacles {
-    const float4 *sph, *cap, *zcap, *cub, *zcub;
+    const float4 *sph, *cap, *zcap, *cub, *zcub, *ball;
     int n_sph, n_cap, n_zcap, n_cub, n_zcub;
 
     __device__ void bind(const SceneHeader &h, const float4 *payload) {
@@ -53,28 +56,20 @@ struct Obstacles {
         zcap = cap + 2 * n_cap;
         cub = zcap + 2 * n_zcap;
         zcub = cub + 4 * n_cub;
+        ball = zcub + 4 * n_zcub;
     }
-
-    // Share `part` of 2^shift: a contiguous share of every table (the shares
-    // of one table partition it), cut by shifts (cheap enough to take at every
-    // obstacle loop instead of holding a sliced copy in registers).
-    __device__ __forceinline__ Obstacles slice_pow2(int part, int shift) const {
-        Obstacles o = *this;
-        cut2(o.sph, o.n_sph, 1, part, shift);
-        cut2(o.cap, o.n_cap, 2, part, shift);
-        cut2(o.zcap, o.n_zcap, 2, part, shift);
-        cut2(o.cub, o.n_cub, 4, part, shift);
-        cut2(o.zcub, o.n_zcub, 4, part, shift);
-        return o;
-    }
-
-private:
-    __device__ static void cut2(const float4 *&p, int &n, int stride, int part, int shift) {
-        const int lo = (n * part) >> shift, hi = (n * (part + 1)) >> shift;
-        p += (size_t)lo * stride;
-        n = hi - lo;
-    }
+    __device__ __forceinline__ int count() const { return n_sph + n_cap + n_zcap + n_cub + n_zcub; }
 };
+
+// Part `part` of 2^shift of a scene's obstacles: i with i mod 2^shift ==
+// part.  Planner waves that share a pass's poses each take one.
+struct Share {
+    int part = 0, shift = 0;
+};
+
+// LDS float4 of a staged scene: its tables (scene_f4) and the balls, at most
+// one per two float4 of tables (every obstacle but a sphere has two or more).
+__host__ __device__ constexpr int scene_lds_f4(int scene_f4) { return scene_f4 + scene_f4 / 2; }
 
 // Read a packed scene's header.  `cap_f4` is the payload size the host
 // allocated; a header that does not fit it (or is inconsistent) is read as an
@@ -89,40 +84,54 @@ __device__ inline void read_header(const float *packed, int cap_f4, SceneHeader 
     if (!ok) h = SceneHeader{0, 0, 0, 0, 0, 0, 0, 0};
 }
 
-// Copy a packed scene's payload into LDS; every lane of the workgroup helps.
+__device__ __forceinline__ float sq3(float dx, float dy, float dz) {
+#pragma clang fp contract(off)
+    return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+}
+
+// Radius of the ball about a segment's midpoint that holds the capsule:
+// |v|/2 + r, padded by 2^-16 relative and 1 mm absolute.  The pad covers the
+// rounding of sqrtf and of the tests it replaces many times over.
+__device__ __forceinline__ float capsule_ball_radius(float vx, float vy, float vz, float r) {
+#pragma clang fp contract(off)
+    return fmaf(0.5f * sqrtf(sq3(vx, vy, vz)) + r, 1.0f + 0x1p-16f, 1e-3f);
+}
+
+// Copy a packed scene's payload into LDS and append the balls
+// (scene_lds_f4(cap_f4) float4 in all); every lane of the workgroup helps.
 __device__ inline void stage_scene(const float *packed, int cap_f4, float4 *lds, SceneHeader &h) {
+#pragma clang fp contract(off)
     read_header(packed, cap_f4, h);
     const float4 *src = reinterpret_cast<const float4 *>(packed) + 2;
     for (int i = threadIdx.x; i < h.n_f4; i += blockDim.x) lds[i] = src[i];
+    const float4 *cap = src + h.n_sph, *cub = cap + 2 * (h.n_cap + h.n_zcap);
+    const int n_caps = h.n_cap + h.n_zcap, n_balls = n_caps + h.n_cub + h.n_zcub;
+    for (int i = threadIdx.x; i < n_balls; i += blockDim.x) {
+        float4 b;
+        if (i < n_caps) {
+            const float4 p = cap[2 * i];
+            float4 v = cap[2 * i + 1];
+            if (i >= h.n_cap) v.x = v.y = 0.0f;   // a z-capsule's test reads v.z alone
+            b = make_float4(fmaf(0.5f, v.x, p.x), fmaf(0.5f, v.y, p.y), fmaf(0.5f, v.z, p.z),
+                            capsule_ball_radius(v.x, v.y, v.z, p.w));
+        } else {
+            const float4 *row = cub + 4 * (i - n_caps);
+            b = row[0];
+            b.w = row[3].w;   // the cull radius of the host pack
+        }
+        lds[h.n_f4 + i] = b;
+    }
     __syncthreads();
 }
 
-// Bind a packed scene for a workgroup: staged into LDS, or read in place.
-template <bool LDS>
+// Stage a packed scene for a workgroup.
 __device__ inline void bind_scene(const float *packed, int cap_f4, float4 *lds, Obstacles &obs) {
     SceneHeader h;
-    if (LDS) {
-        stage_scene(packed, cap_f4, lds, h);
-        obs.bind(h, lds);
-    } else {
-        read_header(packed, cap_f4, h);
-        obs.bind(h, reinterpret_cast<const float4 *>(packed) + 2);
-    }
+    stage_scene(packed, cap_f4, lds, h);
+    obs.bind(h, lds);
 }
 
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
-
-// sphere_environment_in_collision (utils.cuh:211-242) for N spheres per lane
-// at once: OR over the five tables, each obstacle read once (an LDS
-// broadcast: every lane reads the same address) and tested against all N
-// spheres.  Tests are the reference's squared forms (utils.cuh:58-208),
-// value < 0 meaning collision.  With EARLY the wavefront leaves the loops as
-// soon as every active lane has a hit in one of its N spheres.
-//
-// Rounding is pinned: every multiply-add below is an explicit fmaf in a fixed
-// association (and contraction is off), so the CPU oracle can reproduce each
-// verdict bit for bit in its "fused" mode.
-__device__ __forceinline__ float sq3(float dx, float dy, float dz) { return fmaf(dx, dx, fmaf(dy, dy, dz * dz)); }
 
 // Obstacle table read.  LOCAL: the tables are known to be staged in LDS, so
 // the generic pointer is narrowed to an LDS address (its low 32 bits) and
@@ -141,130 +150,298 @@ __device__ __forceinline__ float4 ld_obs(const float4 *p) {
     }
 }
 
-// GROUP: the N spheres all lie inside the ball (gx, gy, gz; gr) on every
-// lane -- the leaves of one link, bounded about the link's gate centre with a
-// 1 mm pad by the generator.  An obstacle whose own bounding ball (sphere:
-// itself; cuboid, capsule: the cull balls below) stays outside that ball on
-// every lane is at least 1 mm from every one of the N spheres, so all N of
-// its tests are positive and the wave skips the obstacle with one test.
-//
-// ANY: only whether some of the N spheres hits is wanted (a leaf group, whose
-// hits the caller ORs): one running minimum over all N spheres replaces the N
-// per-sphere minima (some value < 0 iff their minimum is), which frees N - 1
-// registers of every leaf group; hit[0] carries the answer.
-template <int N, bool EARLY, bool LOCAL = false, bool GROUP = false, bool ANY = false>
-__device__ __forceinline__ void env_multi(const Obstacles &o, const float (&x)[N], const float (&y)[N],
-                                          const float (&z)[N], const float (&r)[N], bool (&hit)[ANY ? 1 : N],
-                                          float gx = 0.0f, float gy = 0.0f, float gz = 0.0f, float gr = 0.0f) {
+// ---- broad phase -----------------------------------------------------------
+// The poses of one wave lie close together (one edge, or neighbouring
+// sub-edges of a chain), so a robot sphere's 64 positions fit a small ball.
+// Before any exact test the wave forms that ball and tests it against 64
+// obstacles at once, one obstacle per lane; the ballot is the list of
+// obstacles any lane can touch.  The exact tests then run over that list
+// alone, with scalar control flow.  Measured against a cull and a branch per
+// sphere and obstacle (the form before; a free 64-pose Panda pass took 9.4k
+// VALU instructions and 975 branches, and a wave alone on its SIMD spent half
+// its cycles waiting on ballot-to-branch chains): 1M C1 edges 17.5 -> 8.2 ms,
+// 10k free Fetch edges 220 -> 95 us, 64 Panda edges 50 -> 26 us, an uneven
+// batch of 128 problems 270 -> 219 ms, the same verdicts bit for bit.
+
+// Largest value over the wave (unsigned order), on every lane.  All 64 lanes
+// must be active.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#define PRRTC_DPP_MAX(CTRL, ROWS)                                                                        \
+    {                                                                                                    \
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);     \
+        v = v > o ? v : o;                                                                               \
+    }
+    PRRTC_DPP_MAX(0x111, 0xf)   // row_shr:1, 2, 4, 8: lane 15 of a row holds the row's
+    PRRTC_DPP_MAX(0x112, 0xf)
+    PRRTC_DPP_MAX(0x114, 0xf)
+    PRRTC_DPP_MAX(0x118, 0xf)
+    PRRTC_DPP_MAX(0x142, 0xa)   // row_bcast:15 into rows 1 and 3
+    PRRTC_DPP_MAX(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
+#undef PRRTC_DPP_MAX
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// A ball that holds one point per live lane; the same on every lane.
+struct WaveBall {
+    float x, y, z, r;
+};
+
+// Centre of the ball: midway between the first and the last live lane's
+// point (the ends of the wave's stretch of the path).
+__device__ __forceinline__ WaveBall ball_centre(float x, float y, float z, uint64_t live) {
 #pragma clang fp contract(off)
-    auto group_far = [&](float cx, float cy, float cz, float cr) {
-        const float rb = gr + cr;
-        return ballot(!(sq3(cx - gx, cy - gy, cz - gz) > rb * rb)) == 0;
-    };
-    // Each sphere keeps the smallest test value over the obstacles seen: some
-    // value < 0 (a collision) iff the minimum is < 0.  One v_min per test
-    // replaces a compare, a select and the bit packing of a boolean OR; a
-    // NaN test value is dropped by fminf as it would fail `< 0`.
-    constexpr int M = ANY ? 1 : N;   // running minima kept
-    float m[M];
-#pragma unroll
-    for (int n = 0; n < M; n++) m[n] = __builtin_huge_valf();
-    auto done = [&]() {
-        bool any_hit = false;
-#pragma unroll
-        for (int n = 0; n < M; n++) any_hit |= m[n] < 0.0f;
-        return ballot(!any_hit) == 0;
-    };
-    auto finish = [&]() {
-#pragma unroll
-        for (int n = 0; n < M; n++) hit[n] = m[n] < 0.0f;
-    };
-    for (int i = 0; i < o.n_sph; i++) {                       // utils.cuh:58-81
+    const int a = __builtin_ctzll(live), b = 63 - __builtin_clzll(live);
+    return WaveBall{0.5f * (lane_value(x, a) + lane_value(x, b)), 0.5f * (lane_value(y, a) + lane_value(y, b)),
+                    0.5f * (lane_value(z, a) + lane_value(z, b)), 0.0f};
+}
+
+// Radius from the live lanes' squared distances: padded by 2^-16 relative,
+// far above the rounding of the distances and of the raw square root (1
+// ulp).  The maximum is taken over the bit patterns, where a NaN is above
+// every number: a lane without a position then makes the radius NaN, and a
+// NaN ball is near every obstacle (in_reach).
+__device__ __forceinline__ float ball_radius(float d2, bool live) {
+#pragma clang fp contract(off)
+    const uint32_t m = wave_max(live ? (uint32_t)__float_as_int(d2) : 0u);
+    return __builtin_amdgcn_sqrtf(__int_as_float((int)m)) * (1.0f + 0x1p-16f);
+}
+
+// Point (x, y, z) of every live lane in one ball (`live`: the ballot of the
+// live lanes, not empty).  All 64 lanes call it.
+__device__ __forceinline__ WaveBall wave_ball(float x, float y, float z, bool on, uint64_t live) {
+#pragma clang fp contract(off)
+    WaveBall c = ball_centre(x, y, z, live);
+    c.r = ball_radius(sq3(x - c.x, y - c.y, z - c.z), on);
+    return c;
+}
+
+// One obstacle's ball on each lane: obstacle i of the scene.  A sphere's is
+// padded like the others (2^-16 relative, 1 mm).
+template <bool LOCAL>
+__device__ __forceinline__ float4 obstacle_ball(const Obstacles &o, int i) {
+#pragma clang fp contract(off)
+    const bool s = i < o.n_sph;
+    float4 b = ld_obs<LOCAL>(s ? o.sph + i : o.ball + (i - o.n_sph));
+    if (s) b.w = fmaf(fabsf(b.w), 1.0f + 0x1p-16f, 1e-3f);
+    return b;
+}
+
+// Whether anything within `reach` of the ball's centre can touch the
+// obstacle ball `b`.  Both radii are padded, so an obstacle out of reach is
+// at least about 1 mm from every live lane's sphere: its exact test would be
+// positive, and skipping it cannot change a verdict.  NaN counts as in reach.
+__device__ __forceinline__ bool in_reach(const float4 &b, const WaveBall &c, float reach) {
+#pragma clang fp contract(off)
+    const float rb = reach + b.w;
+    return !(sq3(b.x - c.x, b.y - c.y, b.z - c.z) > rb * rb);
+}
+
+// ---- exact tests -----------------------------------------------------------
+// The reference's squared forms (utils.cuh:58-208): value < 0 means
+// collision.  Rounding is pinned: every multiply-add is an explicit fmaf in a
+// fixed association (and contraction is off), so the CPU oracle can reproduce
+// each verdict bit for bit in its "fused" mode.
+
+__device__ __forceinline__ float sphere_test(const float4 &s, float x, float y, float z, float r) {   // utils.cuh:58-81
+#pragma clang fp contract(off)
+    const float rs = s.w + r;
+    return fmaf(-rs, rs, sq3(s.x - x, s.y - y, s.z - z));
+}
+__device__ __forceinline__ float capsule_test(const float4 &p, const float4 &v, float x, float y, float z,
+                                              float r) {                                                // utils.cuh:113-126
+#pragma clang fp contract(off)
+    const float dot = fmaf(x - p.x, v.x, fmaf(y - p.y, v.y, (z - p.z) * v.z));
+    const float cdf = fmaxf(fminf(dot * v.w, 1.0f), 0.0f);
+    const float rs = r + p.w;
+    return fmaf(-rs, rs, sq3(x - fmaf(v.x, cdf, p.x), y - fmaf(v.y, cdf, p.y), z - fmaf(v.z, cdf, p.z)));
+}
+__device__ __forceinline__ float z_capsule_test(const float4 &p, const float4 &v, float x, float y, float z,
+                                                float r) {                                              // utils.cuh:135-148
+#pragma clang fp contract(off)
+    const float dot = (z - p.z) * v.z;
+    const float cdf = fmaxf(fminf(dot * v.w, 1.0f), 0.0f);
+    const float rs = r + p.w;
+    return fmaf(-rs, rs, sq3(x - p.x, y - p.y, z - fmaf(v.z, cdf, p.z)));
+}
+__device__ __forceinline__ float cuboid_test(const float4 &c, const float4 &a1, const float4 &a2, const float4 &a3,
+                                             float x, float y, float z, float r) {                      // utils.cuh:158-175
+#pragma clang fp contract(off)
+    const float xs = x - c.x, ys = y - c.y, zs = z - c.z;
+    const float d1 = fmaxf(0.0f, fabsf(fmaf(a1.x, xs, fmaf(a1.y, ys, a1.z * zs))) - c.w);
+    const float d2 = fmaxf(0.0f, fabsf(fmaf(a2.x, xs, fmaf(a2.y, ys, a2.z * zs))) - a1.w);
+    const float d3 = fmaxf(0.0f, fabsf(fmaf(a3.x, xs, fmaf(a3.y, ys, a3.z * zs))) - a2.w);
+    return fmaf(-r, r, sq3(d1, d2, d3));
+}
+__device__ __forceinline__ float z_cuboid_test(const float4 &c, const float4 &a1, const float4 &a2, float x, float y,
+                                               float z, float r) {                                      // utils.cuh:184-201
+#pragma clang fp contract(off)
+    const float xs = x - c.x, ys = y - c.y, zs = z - c.z;
+    const float d1 = fmaxf(0.0f, fabsf(fmaf(a1.x, xs, a1.y * ys)) - c.w);
+    const float d2 = fmaxf(0.0f, fabsf(fmaf(a2.x, xs, a2.y * ys)) - a1.w);
+    const float d3 = fmaxf(0.0f, fabsf(zs) - a2.w);
+    return fmaf(-r, r, sq3(d1, d2, d3));
+}
+
+// Smallest test value of obstacle i (wave-uniform) against N spheres per
+// lane, lowered into m[n] (ANY: into m[0], for callers that want only
+// whether some sphere hits).  A NaN test value is dropped by fminf as it
+// would fail `< 0`.  With CULL each sphere first asks whether any lane is
+// within reach of the obstacle's ball: of the N spheres of a link near an
+// obstacle most are not, and the exact test costs three times as much.
+template <int N, bool LOCAL, bool ANY, bool CULL>
+__device__ __forceinline__ void test_obstacle(const Obstacles &o, int i, const float *x, const float *y,
+                                              const float *z, const float *r, float *m) {
+#pragma clang fp contract(off)
+    if (i < o.n_sph) {
         const float4 s = ld_obs<LOCAL>(o.sph + i);
-        if (GROUP && group_far(s.x, s.y, s.z, s.w)) continue;
 #pragma unroll
-        for (int n = 0; n < N; n++) {
-            const float rs = s.w + r[n];
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], fmaf(-rs, rs, sq3(s.x - x[n], s.y - y[n], s.z - z[n])));
-        }
-        if (EARLY && (i & 7) == 7 && done()) return finish();
+        for (int n = 0; n < N; n++) m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], sphere_test(s, x[n], y[n], z[n], r[n]));
+        return;
     }
-    if (EARLY && o.n_sph && done()) return finish();
-    // Capsules are culled like cuboids (below) against the ball about the
-    // segment's midpoint that holds the capsule: radius |v|/2 + r, padded by
-    // 2^-16 relative and 1 mm absolute.  The pad covers the rounding of
-    // sqrtf and of both tests many times over.
-    for (int i = 0; i < o.n_cap; i++) {                       // utils.cuh:113-126
+    i -= o.n_sph;
+    float4 b;
+    if constexpr (CULL) b = ld_obs<LOCAL>(o.ball + i);
+    auto far = [&](int n) {
+#pragma clang fp contract(off)
+        if constexpr (CULL) {
+            const float rb = r[n] + b.w;
+            return ballot(!(sq3(x[n] - b.x, y[n] - b.y, z[n] - b.z) > rb * rb)) == 0;
+        } else {
+            return false;
+        }
+    };
+    if (i < o.n_cap) {
         const float4 p = ld_obs<LOCAL>(o.cap + 2 * i), v = ld_obs<LOCAL>(o.cap + 2 * i + 1);
-        const float mx = fmaf(0.5f, v.x, p.x), my = fmaf(0.5f, v.y, p.y), mz = fmaf(0.5f, v.z, p.z);
-        const float cull = fmaf(0.5f * sqrtf(sq3(v.x, v.y, v.z)) + p.w, 1.0f + 0x1p-16f, 1e-3f);
-        if (GROUP && group_far(mx, my, mz, cull)) continue;
 #pragma unroll
         for (int n = 0; n < N; n++) {
-            const float rb = r[n] + cull;
-            if (ballot(!(sq3(x[n] - mx, y[n] - my, z[n] - mz) > rb * rb)) == 0) continue;
-            const float dot = fmaf(x[n] - p.x, v.x, fmaf(y[n] - p.y, v.y, (z[n] - p.z) * v.z));
-            const float cdf = fmaxf(fminf(dot * v.w, 1.0f), 0.0f);
-            const float rs = r[n] + p.w;
-            const float d = sq3(x[n] - fmaf(v.x, cdf, p.x), y[n] - fmaf(v.y, cdf, p.y), z[n] - fmaf(v.z, cdf, p.z));
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], fmaf(-rs, rs, d));
+            if (far(n)) continue;
+            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], capsule_test(p, v, x[n], y[n], z[n], r[n]));
         }
-        if (EARLY && (i & 7) == 7 && done()) return finish();
+        return;
     }
-    if (EARLY && o.n_cap && done()) return finish();
-    for (int i = 0; i < o.n_zcap; i++) {                      // utils.cuh:135-148
+    i -= o.n_cap;
+    if (i < o.n_zcap) {
         const float4 p = ld_obs<LOCAL>(o.zcap + 2 * i), v = ld_obs<LOCAL>(o.zcap + 2 * i + 1);
 #pragma unroll
-        for (int n = 0; n < N; n++) {
-            const float dot = (z[n] - p.z) * v.z;
-            const float cdf = fmaxf(fminf(dot * v.w, 1.0f), 0.0f);
-            const float rs = r[n] + p.w;
-            const float d = sq3(x[n] - p.x, y[n] - p.y, z[n] - fmaf(v.z, cdf, p.z));
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], fmaf(-rs, rs, d));
-        }
-        if (EARLY && (i & 7) == 7 && done()) return finish();
+        for (int n = 0; n < N; n++)
+            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], z_capsule_test(p, v, x[n], y[n], z[n], r[n]));
+        return;
     }
-    if (EARLY && o.n_zcap && done()) return finish();
-    // Cuboids carry a cull radius (a3.w): the box's half-diagonal with a 1 mm
-    // pad, from the host pack.  When no lane's sphere comes within r + cull
-    // of the centre, the box test is positive by at least that pad on every
-    // lane and cannot lower m below 0, so the wave skips it (the test itself,
-    // where it runs, is unchanged).
-    for (int i = 0; i < o.n_cub; i++) {                       // utils.cuh:158-175
+    i -= o.n_zcap;
+    if (i < o.n_cub) {
         const float4 c = ld_obs<LOCAL>(o.cub + 4 * i), a1 = ld_obs<LOCAL>(o.cub + 4 * i + 1),
                      a2 = ld_obs<LOCAL>(o.cub + 4 * i + 2), a3 = ld_obs<LOCAL>(o.cub + 4 * i + 3);
-        if (GROUP && group_far(c.x, c.y, c.z, a3.w)) continue;
 #pragma unroll
         for (int n = 0; n < N; n++) {
-            const float xs = x[n] - c.x, ys = y[n] - c.y, zs = z[n] - c.z;
-            const float rb = r[n] + a3.w;
-            if (ballot(!(sq3(xs, ys, zs) > rb * rb)) == 0) continue;
-            const float d1 = fmaxf(0.0f, fabsf(fmaf(a1.x, xs, fmaf(a1.y, ys, a1.z * zs))) - c.w);
-            const float d2 = fmaxf(0.0f, fabsf(fmaf(a2.x, xs, fmaf(a2.y, ys, a2.z * zs))) - a1.w);
-            const float d3 = fmaxf(0.0f, fabsf(fmaf(a3.x, xs, fmaf(a3.y, ys, a3.z * zs))) - a2.w);
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], fmaf(-r[n], r[n], sq3(d1, d2, d3)));
+            if (far(n)) continue;
+            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], cuboid_test(c, a1, a2, a3, x[n], y[n], z[n], r[n]));
         }
-        if (EARLY && (i & 7) == 7 && done()) return finish();
+        return;
     }
-    if (EARLY && o.n_cub && done()) return finish();
-    for (int i = 0; i < o.n_zcub; i++) {                      // utils.cuh:184-201
-        const float4 c = ld_obs<LOCAL>(o.zcub + 4 * i), a1 = ld_obs<LOCAL>(o.zcub + 4 * i + 1),
-                     a2 = ld_obs<LOCAL>(o.zcub + 4 * i + 2);
-        const float cull = ld_obs<LOCAL>(o.zcub + 4 * i + 3).w;
-        if (GROUP && group_far(c.x, c.y, c.z, cull)) continue;
+    i -= o.n_cub;
+    const float4 c = ld_obs<LOCAL>(o.zcub + 4 * i), a1 = ld_obs<LOCAL>(o.zcub + 4 * i + 1),
+                 a2 = ld_obs<LOCAL>(o.zcub + 4 * i + 2);
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        if (far(n)) continue;
+        m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], z_cuboid_test(c, a1, a2, x[n], y[n], z[n], r[n]));
+    }
+}
+
+// sphere_environment_in_collision (utils.cuh:211-242) for N spheres per
+// lane, whose answer is wanted sphere by sphere: hit[n] on each live lane.
+// All 64 lanes call it; `on` marks the live ones (at least one).
+template <int N, bool LOCAL>
+__device__ __forceinline__ void env_hits(const Obstacles &o, Share sh, const float (&x)[N], const float (&y)[N],
+                                         const float (&z)[N], const float (&r)[N], bool on, bool (&hit)[N]) {
+#pragma clang fp contract(off)
+    const uint64_t live = ballot(on);
+    const int lane = threadIdx.x & (kWave - 1);
+    const int mine = (o.count() - sh.part + (1 << sh.shift) - 1) >> sh.shift;   // obstacles of the share
+    float m[N];
+#pragma unroll
+    for (int n = 0; n < N; n++) m[n] = __builtin_huge_valf();
+    for (int base = 0; base < mine; base += kWave) {
+        const int j = base + lane;
+        const bool have = j < mine;
+        const float4 b = obstacle_ball<LOCAL>(o, have ? (j << sh.shift) + sh.part : 0);
+        uint64_t near[N];
 #pragma unroll
         for (int n = 0; n < N; n++) {
-            const float xs = x[n] - c.x, ys = y[n] - c.y, zs = z[n] - c.z;
-            const float rb = r[n] + cull;
-            if (ballot(!(sq3(xs, ys, zs) > rb * rb)) == 0) continue;
-            const float d1 = fmaxf(0.0f, fabsf(fmaf(a1.x, xs, a1.y * ys)) - c.w);
-            const float d2 = fmaxf(0.0f, fabsf(fmaf(a2.x, xs, a2.y * ys)) - a1.w);
-            const float d3 = fmaxf(0.0f, fabsf(zs) - a2.w);
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], fmaf(-r[n], r[n], sq3(d1, d2, d3)));
+            const WaveBall c = wave_ball(x[n], y[n], z[n], on, live);
+            near[n] = ballot(have && in_reach(b, c, c.r + r[n]));
         }
-        if (EARLY && (i & 7) == 7 && done()) return finish();
+#pragma unroll
+        for (int n = 0; n < N; n++) {
+            for (uint64_t w = near[n]; w; w &= w - 1) {
+                const int i = __builtin_amdgcn_readfirstlane(((base + __builtin_ctzll(w)) << sh.shift) + sh.part);
+                test_obstacle<1, LOCAL, false, false>(o, i, x + n, y + n, z + n, r + n, m + n);
+            }
+        }
     }
-    finish();
+#pragma unroll
+    for (int n = 0; n < N; n++) hit[n] = m[n] < 0.0f;
+}
+
+// Whether any of N spheres (the leaves of one link) hits an obstacle, on each
+// live lane.  The spheres of every lane lie in one ball about `c`, `reach`
+// its radius.  One running minimum serves the group (some value < 0 iff their
+// minimum is).  EARLY: the wave leaves once every live lane has a hit.
+template <int N, bool EARLY, bool LOCAL>
+__device__ __forceinline__ bool env_group(const Obstacles &o, Share sh, const float (&x)[N], const float (&y)[N],
+                                          const float (&z)[N], const float (&r)[N], bool on, const WaveBall &c,
+                                          float reach) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & (kWave - 1);
+    const int mine = (o.count() - sh.part + (1 << sh.shift) - 1) >> sh.shift;
+    float m[1] = {__builtin_huge_valf()};
+    for (int base = 0; base < mine; base += kWave) {
+        const int j = base + lane;
+        const bool have = j < mine;
+        const float4 b = obstacle_ball<LOCAL>(o, have ? (j << sh.shift) + sh.part : 0);
+        for (uint64_t w = ballot(have && in_reach(b, c, reach)); w; w &= w - 1) {
+            const int i = __builtin_amdgcn_readfirstlane(((base + __builtin_ctzll(w)) << sh.shift) + sh.part);
+            test_obstacle<N, LOCAL, true, true>(o, i, x, y, z, r, m);
+            if (EARLY && ballot(on && !(m[0] < 0.0f)) == 0) return true;
+        }
+    }
+    return m[0] < 0.0f;
+}
+
+// env_group for spheres without a bound of their own: the ball is taken
+// about the first sphere's stretch and holds all of them.
+template <int N, bool EARLY, bool LOCAL>
+__device__ __forceinline__ bool env_leaves(const Obstacles &o, Share sh, const float (&x)[N], const float (&y)[N],
+                                           const float (&z)[N], const float (&r)[N], bool on) {
+#pragma clang fp contract(off)
+    WaveBall c = ball_centre(x[0], y[0], z[0], ballot(on));
+    uint32_t d = 0;
+    float rmax = 0.0f;
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        // bit patterns of non-negative floats order like the floats, a NaN above all
+        const uint32_t e = (uint32_t)__float_as_int(sq3(x[n] - c.x, y[n] - c.y, z[n] - c.z));
+        d = e > d ? e : d;
+        rmax = fmaxf(rmax, r[n]);
+    }
+    c.r = ball_radius(__int_as_float((int)d), on);
+    return env_group<N, EARLY, LOCAL>(o, sh, x, y, z, r, on, c, c.r + rmax);
+}
+
+// env_group for spheres that lie in the ball (gx, gy, gz; gr) on every lane
+// -- the leaves of one link, bounded about the link's gate centre with a
+// 1 mm pad by the generator.
+template <int N, bool EARLY, bool LOCAL>
+__device__ __forceinline__ bool env_leaves_bounded(const Obstacles &o, Share sh, const float (&x)[N],
+                                                   const float (&y)[N], const float (&z)[N], const float (&r)[N],
+                                                   bool on, float gx, float gy, float gz, float gr) {
+#pragma clang fp contract(off)
+    const WaveBall c = wave_ball(gx, gy, gz, on, ballot(on));
+    return env_group<N, EARLY, LOCAL>(o, sh, x, y, z, r, on, c, c.r + gr);
 }
 
 // sphere_sphere_self_collision (utils.cuh:83-86) with the radius sum folded.
@@ -297,31 +474,27 @@ struct CheckCtx {
     // Self-collision group j (numbered in check order) is this wave's to
     // test; a lone wave tests every group.
     __device__ __forceinline__ bool mine(int) const { return true; }
-    template <int N, bool EARLY>
-    __device__ __forceinline__ void env_multi(const float (&x)[N], const float (&y)[N], const float (&z)[N],
+    // N gate spheres against the obstacles, hit[n] on each live lane; called
+    // by the whole wave while some lane is live.
+    template <int N>
+    __device__ __forceinline__ void env_gates(const float (&x)[N], const float (&y)[N], const float (&z)[N],
                                               const float (&r)[N], bool (&hit)[N]) const {
-        prrtc::env_multi<N, EARLY>(obs, x, y, z, r, hit);
+        env_hits<N, false>(obs, Share{}, x, y, z, r, live(), hit);
     }
-    // Whether any of the N spheres hits an obstacle (a leaf group).
+    // Whether any of the N spheres of a leaf group hits an obstacle, on the
+    // lanes with `on` (at least one); called by the whole wave.
     template <int N, bool EARLY>
     __device__ __forceinline__ bool env_any(const float (&x)[N], const float (&y)[N], const float (&z)[N],
-                                            const float (&r)[N]) const {
-        bool h[1];
-        prrtc::env_multi<N, EARLY, false, false, true>(obs, x, y, z, r, h);
-        return h[0];
+                                            const float (&r)[N], bool on) const {
+        return env_leaves<N, EARLY, false>(obs, Share{}, x, y, z, r, on);
     }
     // The same for N spheres that lie inside the ball (gx, gy, gz; gr) on
-    // every lane: an obstacle whose bounding ball stays outside it is skipped
-    // for the whole group (GROUP).  With one running minimum per group the
-    // bound fits the one-wave-per-edge kernels' register budget (Panda 209
-    // VGPRs, Fetch 255: two waves per SIMD, no scratch).
+    // every lane.
     template <int N, bool EARLY>
     __device__ __forceinline__ bool env_any_bounded(const float (&x)[N], const float (&y)[N], const float (&z)[N],
-                                                    const float (&r)[N], float gx, float gy, float gz,
+                                                    const float (&r)[N], bool on, float gx, float gy, float gz,
                                                     float gr) const {
-        bool h[1];
-        prrtc::env_multi<N, EARLY, false, true, true>(obs, x, y, z, r, h, gx, gy, gz, gr);
-        return h[0];
+        return env_leaves_bounded<N, EARLY, false>(obs, Share{}, x, y, z, r, on, gx, gy, gz, gr);
     }
     __device__ __forceinline__ bool self(float ax, float ay, float az, float bx, float by, float bz, float rs) const {
         return self_hit(ax, ay, az, bx, by, bz, rs);
@@ -356,9 +529,9 @@ struct SphereRobot {     // Robots.hh:190-237; fkcc<Sphere>, utils.cuh:330-334
     __device__ __forceinline__ static void check(const float *q, Ctx &ctx) {
         const float x[1] = {q[0]}, y[1] = {q[1]}, z[1] = {q[2]}, r[1] = {1.0f};
         bool h[1];
-        if (ctx.live()) {
-            ctx.template env_multi<1, false>(x, y, z, r, h);
-            if (h[0]) ctx.hit();
+        if (ctx.any(ctx.live())) {
+            ctx.template env_gates<1>(x, y, z, r, h);
+            if (ctx.live() && h[0]) ctx.hit();
         }
         ctx.stop();
     }

@@ -70,9 +70,8 @@ struct TaskCtx : CheckCtx {
     int pass;         // index of the current pass within the task
     int waves;        // waves sharing this pass's poses (1: the wave has poses of its own)
     int gbase;        // first wave of those
-    // this wave's share of the obstacles: part `part` of 2^shift (obs holds
-    // the whole staged scene; the share is cut at every obstacle loop)
-    int part, shift;
+    // this wave's share of the obstacles (obs holds the whole staged scene)
+    Share share;
     bool shared_stop; // the task runs on several waves: stop keys go through LDS
     bool wide_ok;     // its chain passes may give each wave poses of its own
     unsigned mine12;  // bit i: self groups j with j mod 12 == i are this wave's (12 = lcm of 1..4)
@@ -90,25 +89,21 @@ struct TaskCtx : CheckCtx {
     static_assert(kMaxTaskWaves <= 4, "the 12-group pattern of mine12 needs 12 % waves == 0");
     __device__ __forceinline__ bool mine(int j) const { return (mine12 >> (j % 12)) & 1u; }
     // The obstacle tables of a task are always staged in LDS.
-    template <int N, bool EARLY>
-    __device__ __forceinline__ void env_multi(const float (&x)[N], const float (&y)[N], const float (&z)[N],
+    template <int N>
+    __device__ __forceinline__ void env_gates(const float (&x)[N], const float (&y)[N], const float (&z)[N],
                                               const float (&r)[N], bool (&hit)[N]) const {
-        prrtc::env_multi<N, EARLY, true>(obs.slice_pow2(part, shift), x, y, z, r, hit);
+        env_hits<N, true>(obs, share, x, y, z, r, live(), hit);
     }
     template <int N, bool EARLY>
     __device__ __forceinline__ bool env_any(const float (&x)[N], const float (&y)[N], const float (&z)[N],
-                                            const float (&r)[N]) const {
-        bool h[1];
-        prrtc::env_multi<N, EARLY, true, false, true>(obs.slice_pow2(part, shift), x, y, z, r, h);
-        return h[0];
+                                            const float (&r)[N], bool on) const {
+        return env_leaves<N, EARLY, true>(obs, share, x, y, z, r, on);
     }
     template <int N, bool EARLY>
     __device__ __forceinline__ bool env_any_bounded(const float (&x)[N], const float (&y)[N], const float (&z)[N],
-                                                    const float (&r)[N], float gx, float gy, float gz,
+                                                    const float (&r)[N], bool on, float gx, float gy, float gz,
                                                     float gr) const {
-        bool h[1];
-        prrtc::env_multi<N, EARLY, true, true, true>(obs.slice_pow2(part, shift), x, y, z, r, h, gx, gy, gz, gr);
-        return h[0];
+        return env_leaves_bounded<N, EARLY, true>(obs, share, x, y, z, r, on, gx, gy, gz, gr);
     }
     // CheckCtx::stop in path mode (a planner task is never in pose mode),
     // with the stop key shared across waves.
@@ -170,8 +165,8 @@ __device__ __attribute__((always_inline)) void plan_task(const PlanDesc &d, Plan
         const int gs = tm.waves / G;          // waves per group
         gw = tm.wave / gs;
         const int wi = tm.wave - gw * gs;     // this wave's index in its group
-        ctx.part = wi;
-        ctx.shift = gs == 4 ? 2 : gs == 2 ? 1 : 0;
+        ctx.share.part = wi;
+        ctx.share.shift = gs == 4 ? 2 : gs == 2 ? 1 : 0;
         ctx.waves = gs;
         ctx.gbase = gw * gs;
         unsigned m = 0;
@@ -863,7 +858,7 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
         const PlanDesc &d = descs[p];
         PlanState *st = states + p;
         if (staged != p) {   // every wave is past its last use of the staged scene
-            bind_scene<true>(d.scene, d.scene_f4, lds, scene_obs);
+            bind_scene(d.scene, d.scene_f4, lds, scene_obs);
             staged = p;
         }
         // Without a crowd claim every wave runs the one slot and checks its
@@ -965,7 +960,7 @@ void k_round_tasks(const PlanDesc *__restrict__ descs, PlanState *states, int ma
     TaskCtx ctx;
     ctx.independent = false;
     ctx.gbuf = gbuf;
-    bind_scene<true>(d.scene, d.scene_f4, lds, ctx.obs);
+    bind_scene(d.scene, d.scene_f4, lds, ctx.obs);
     ctx.wide_ok = false;   // a grid of every running problem's slots: throughput-bound
     plan_task<Robot>(d, st, s, ctx, a, a + (lds_ext + 1) * D, a + (lds_ext + 5) * D,
                      reinterpret_cast<int *>(a + (lds_ext + 5) * D + 2 * kMaxTaskWaves), team_workgroup());
@@ -1403,7 +1398,7 @@ static void start_group(GroupRun &gr, int path_cap) {
     std::vector<size_t> o_block(P);
     int lds_f4 = 0, ext_all = 0;
     for (int i = 0; i < P; i++) {
-        lds_f4 = std::max(lds_f4, (lay[i].scene_floats - 8) / 4);
+        lds_f4 = std::max(lds_f4, scene_lds_f4((lay[i].scene_floats - 8) / 4));
         ext_all = std::max(ext_all, lay[i].max_ext);
         o_block[i] = dl.take(lay[i].bytes);
     }

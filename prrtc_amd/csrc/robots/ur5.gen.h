@@ -123,14 +123,14 @@ template <class Ctx>
 __device__ __forceinline__ void check(const float *q, Ctx &ctx) {
     PRRTC_FK_BODY
     uint64_t gate = 0;  /* bit k: env check k's gate sphere hit */
-    if (ctx.live()) {
+    if (ctx.any(ctx.live())) {
         {
             const float ex[7] = {0.03500000014901161f * R0_01, -0.24285714328289032f * R1_01 + -0.008571428246796131f * R0_01 + t1_0, -0.19870834052562714f * R2_01 + t2_0, 0.02500000037252903f * R0_01 + t3_0, 0.02500000037252903f * M4_02 + t4_0, 0.02500000037252903f * R4_01 + t5_0, 2.449293581093244e-18f * R5_00 + 0.12229999899864197f * R4_01 + t5_0};
             const float ey[7] = {0.03500000014901161f * R0_11, -0.24285714328289032f * R1_11 + -0.008571428246796131f * R0_11 + t1_1, -0.19870834052562714f * R2_11 + t2_1, 0.02500000037252903f * R0_11 + t3_1, 0.02500000037252903f * M4_12 + t4_1, 0.02500000037252903f * R4_11 + t5_1, 2.449293581093244e-18f * R5_10 + 0.12229999899864197f * R4_11 + t5_1};
             const float ez[7] = {0.08915899693965912f, 0.08915899693965912f + -0.24285714328289032f * R1_21, -0.19870834052562714f * R2_21 + t2_2, t3_2, 0.02500000037252903f * M4_22 + t3_2, 0.02500000037252903f * R4_21 + t5_2, 2.449293581093244e-18f * R5_20 + 0.12229999899864197f * R4_21 + t5_2};
             const float er[7] = {0.10999999940395355f, 0.3080083429813385f, 0.2487083375453949f, 0.07000000029802322f, 0.07000000029802322f, 0.06499999761581421f, 0.03999999910593033f};
             bool eh[7];
-            ctx.template env_multi<7, false>(ex, ey, ez, er, eh);
+            ctx.template env_gates<7>(ex, ey, ez, er, eh);
             gate |= ((uint64_t)eh[0] << 0) | ((uint64_t)eh[1] << 1) | ((uint64_t)eh[2] << 2) | ((uint64_t)eh[3] << 3) | ((uint64_t)eh[4] << 4) | ((uint64_t)eh[5] << 5) | ((uint64_t)eh[6] << 6);
         }
     }
@@ -139,85 +139,79 @@ __device__ __forceinline__ void check(const float *q, Ctx &ctx) {
     if (ctx.stop()) return;
     /* env leaves: shoulder_link */
     if (ctx.any(ctx.live() && (gate >> 0 & 1))) {
-        if (ctx.live() && (gate >> 0 & 1)) {
-            {
-                const float ex[2] = {0.0f, 0.07000000029802322f * R0_01};
-                const float ey[2] = {0.0f, 0.07000000029802322f * R0_11};
-                const float ez[2] = {0.08915899693965912f, 0.08915899693965912f};
-                const float er[2] = {0.07500000298023224f, 0.07000000029802322f};
-                const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er);
-                if (eh) ctx.hit();
-            }
+        const bool on = ctx.live() && (gate >> 0 & 1);
+        {
+            const float ex[2] = {0.0f, 0.07000000029802322f * R0_01};
+            const float ey[2] = {0.0f, 0.07000000029802322f * R0_11};
+            const float ez[2] = {0.08915899693965912f, 0.08915899693965912f};
+            const float er[2] = {0.07500000298023224f, 0.07000000029802322f};
+            const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er, on);
+            if (on && eh) ctx.hit();
         }
         if (ctx.stop()) return;
     }
     /* env leaves: upper_arm_link */
     if (ctx.any(ctx.live() && (gate >> 1 & 1))) {
-        if (ctx.live() && (gate >> 1 & 1)) {
-            {
-                const float ex[7] = {t1_0, -0.08500000089406967f * R1_01 + t1_0, -0.17000000178813934f * R1_01 + t1_0, -0.2549999952316284f * R1_01 + t1_0, -0.3400000035762787f * R1_01 + t1_0, -0.42500001192092896f * R1_01 + t1_0, -0.42500001192092896f * R1_01 + -0.05999999865889549f * R0_01 + t1_0};
-                const float ey[7] = {t1_1, -0.08500000089406967f * R1_11 + t1_1, -0.17000000178813934f * R1_11 + t1_1, -0.2549999952316284f * R1_11 + t1_1, -0.3400000035762787f * R1_11 + t1_1, -0.42500001192092896f * R1_11 + t1_1, -0.42500001192092896f * R1_11 + -0.05999999865889549f * R0_11 + t1_1};
-                const float ez[7] = {0.08915899693965912f, 0.08915899693965912f + -0.08500000089406967f * R1_21, 0.08915899693965912f + -0.17000000178813934f * R1_21, 0.08915899693965912f + -0.2549999952316284f * R1_21, 0.08915899693965912f + -0.3400000035762787f * R1_21, 0.08915899693965912f + -0.42500001192092896f * R1_21, 0.08915899693965912f + -0.42500001192092896f * R1_21};
-                const float er[7] = {0.06499999761581421f, 0.054999999701976776f, 0.054999999701976776f, 0.054999999701976776f, 0.054999999701976776f, 0.06499999761581421f, 0.05999999865889549f};
-                const bool eh = ctx.template env_any_bounded<7, true>(ex, ey, ez, er, -0.24285714328289032f * R1_01 + -0.008571428246796131f * R0_01 + t1_0, -0.24285714328289032f * R1_11 + -0.008571428246796131f * R0_11 + t1_1, 0.08915899693965912f + -0.24285714328289032f * R1_21, 0.30901309847831726f);
-                if (eh) ctx.hit();
-            }
+        const bool on = ctx.live() && (gate >> 1 & 1);
+        {
+            const float ex[7] = {t1_0, -0.08500000089406967f * R1_01 + t1_0, -0.17000000178813934f * R1_01 + t1_0, -0.2549999952316284f * R1_01 + t1_0, -0.3400000035762787f * R1_01 + t1_0, -0.42500001192092896f * R1_01 + t1_0, -0.42500001192092896f * R1_01 + -0.05999999865889549f * R0_01 + t1_0};
+            const float ey[7] = {t1_1, -0.08500000089406967f * R1_11 + t1_1, -0.17000000178813934f * R1_11 + t1_1, -0.2549999952316284f * R1_11 + t1_1, -0.3400000035762787f * R1_11 + t1_1, -0.42500001192092896f * R1_11 + t1_1, -0.42500001192092896f * R1_11 + -0.05999999865889549f * R0_11 + t1_1};
+            const float ez[7] = {0.08915899693965912f, 0.08915899693965912f + -0.08500000089406967f * R1_21, 0.08915899693965912f + -0.17000000178813934f * R1_21, 0.08915899693965912f + -0.2549999952316284f * R1_21, 0.08915899693965912f + -0.3400000035762787f * R1_21, 0.08915899693965912f + -0.42500001192092896f * R1_21, 0.08915899693965912f + -0.42500001192092896f * R1_21};
+            const float er[7] = {0.06499999761581421f, 0.054999999701976776f, 0.054999999701976776f, 0.054999999701976776f, 0.054999999701976776f, 0.06499999761581421f, 0.05999999865889549f};
+            const bool eh = ctx.template env_any_bounded<7, true>(ex, ey, ez, er, on, -0.24285714328289032f * R1_01 + -0.008571428246796131f * R0_01 + t1_0, -0.24285714328289032f * R1_11 + -0.008571428246796131f * R0_11 + t1_1, 0.08915899693965912f + -0.24285714328289032f * R1_21, 0.30901309847831726f);
+            if (on && eh) ctx.hit();
         }
         if (ctx.stop()) return;
     }
     /* env leaves: forearm_link */
     if (ctx.any(ctx.live() && (gate >> 2 & 1))) {
-        if (ctx.live() && (gate >> 2 & 1)) {
-            {
-                const float ex[6] = {t2_0, -0.07999999821186066f * R2_01 + t2_0, -0.1599999964237213f * R2_01 + t2_0, -0.23999999463558197f * R2_01 + t2_0, -0.3199999928474426f * R2_01 + t2_0, -0.3922500014305115f * R2_01 + t2_0};
-                const float ey[6] = {t2_1, -0.07999999821186066f * R2_11 + t2_1, -0.1599999964237213f * R2_11 + t2_1, -0.23999999463558197f * R2_11 + t2_1, -0.3199999928474426f * R2_11 + t2_1, -0.3922500014305115f * R2_11 + t2_1};
-                const float ez[6] = {t2_2, -0.07999999821186066f * R2_21 + t2_2, -0.1599999964237213f * R2_21 + t2_2, -0.23999999463558197f * R2_21 + t2_2, -0.3199999928474426f * R2_21 + t2_2, -0.3922500014305115f * R2_21 + t2_2};
-                const float er[6] = {0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f};
-                const bool eh = ctx.template env_any_bounded<6, true>(ex, ey, ez, er, -0.19870834052562714f * R2_01 + t2_0, -0.19870834052562714f * R2_11 + t2_1, -0.19870834052562714f * R2_21 + t2_2, 0.24971213936805725f);
-                if (eh) ctx.hit();
-            }
+        const bool on = ctx.live() && (gate >> 2 & 1);
+        {
+            const float ex[6] = {t2_0, -0.07999999821186066f * R2_01 + t2_0, -0.1599999964237213f * R2_01 + t2_0, -0.23999999463558197f * R2_01 + t2_0, -0.3199999928474426f * R2_01 + t2_0, -0.3922500014305115f * R2_01 + t2_0};
+            const float ey[6] = {t2_1, -0.07999999821186066f * R2_11 + t2_1, -0.1599999964237213f * R2_11 + t2_1, -0.23999999463558197f * R2_11 + t2_1, -0.3199999928474426f * R2_11 + t2_1, -0.3922500014305115f * R2_11 + t2_1};
+            const float ez[6] = {t2_2, -0.07999999821186066f * R2_21 + t2_2, -0.1599999964237213f * R2_21 + t2_2, -0.23999999463558197f * R2_21 + t2_2, -0.3199999928474426f * R2_21 + t2_2, -0.3922500014305115f * R2_21 + t2_2};
+            const float er[6] = {0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f, 0.05000000074505806f};
+            const bool eh = ctx.template env_any_bounded<6, true>(ex, ey, ez, er, on, -0.19870834052562714f * R2_01 + t2_0, -0.19870834052562714f * R2_11 + t2_1, -0.19870834052562714f * R2_21 + t2_2, 0.24971213936805725f);
+            if (on && eh) ctx.hit();
         }
         if (ctx.stop()) return;
     }
     /* env leaves: wrist_1_link */
     if (ctx.any(ctx.live() && (gate >> 3 & 1))) {
-        if (ctx.live() && (gate >> 3 & 1)) {
-            {
-                const float ex[2] = {t3_0, 0.05000000074505806f * R0_01 + t3_0};
-                const float ey[2] = {t3_1, 0.05000000074505806f * R0_11 + t3_1};
-                const float ez[2] = {t3_2, t3_2};
-                const float er[2] = {0.04500000178813934f, 0.04500000178813934f};
-                const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er);
-                if (eh) ctx.hit();
-            }
+        const bool on = ctx.live() && (gate >> 3 & 1);
+        {
+            const float ex[2] = {t3_0, 0.05000000074505806f * R0_01 + t3_0};
+            const float ey[2] = {t3_1, 0.05000000074505806f * R0_11 + t3_1};
+            const float ez[2] = {t3_2, t3_2};
+            const float er[2] = {0.04500000178813934f, 0.04500000178813934f};
+            const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er, on);
+            if (on && eh) ctx.hit();
         }
         if (ctx.stop()) return;
     }
     /* env leaves: wrist_2_link */
     if (ctx.any(ctx.live() && (gate >> 4 & 1))) {
-        if (ctx.live() && (gate >> 4 & 1)) {
-            {
-                const float ex[2] = {t4_0, 0.05000000074505806f * M4_02 + t4_0};
-                const float ey[2] = {t4_1, 0.05000000074505806f * M4_12 + t4_1};
-                const float ez[2] = {t3_2, 0.05000000074505806f * M4_22 + t3_2};
-                const float er[2] = {0.04500000178813934f, 0.04500000178813934f};
-                const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er);
-                if (eh) ctx.hit();
-            }
+        const bool on = ctx.live() && (gate >> 4 & 1);
+        {
+            const float ex[2] = {t4_0, 0.05000000074505806f * M4_02 + t4_0};
+            const float ey[2] = {t4_1, 0.05000000074505806f * M4_12 + t4_1};
+            const float ez[2] = {t3_2, 0.05000000074505806f * M4_22 + t3_2};
+            const float er[2] = {0.04500000178813934f, 0.04500000178813934f};
+            const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er, on);
+            if (on && eh) ctx.hit();
         }
         if (ctx.stop()) return;
     }
     /* env leaves: wrist_3_link */
     if (ctx.any(ctx.live() && (gate >> 5 & 1))) {
-        if (ctx.live() && (gate >> 5 & 1)) {
-            {
-                const float ex[2] = {t5_0, 0.05000000074505806f * R4_01 + t5_0};
-                const float ey[2] = {t5_1, 0.05000000074505806f * R4_11 + t5_1};
-                const float ez[2] = {t5_2, 0.05000000074505806f * R4_21 + t5_2};
-                const float er[2] = {0.03999999910593033f, 0.03999999910593033f};
-                const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er);
-                if (eh) ctx.hit();
-            }
+        const bool on = ctx.live() && (gate >> 5 & 1);
+        {
+            const float ex[2] = {t5_0, 0.05000000074505806f * R4_01 + t5_0};
+            const float ey[2] = {t5_1, 0.05000000074505806f * R4_11 + t5_1};
+            const float ez[2] = {t5_2, 0.05000000074505806f * R4_21 + t5_2};
+            const float er[2] = {0.03999999910593033f, 0.03999999910593033f};
+            const bool eh = ctx.template env_any<2, true>(ex, ey, ez, er, on);
+            if (on && eh) ctx.hit();
         }
         if (ctx.stop()) return;
     }

@@ -32,15 +32,15 @@ __global__ __launch_bounds__(kWave) void k_fk_spheres(const float *__restrict__ 
     Robot::fk_spheres(q, out + (size_t)i * Robot::NSPHERES * 3);
 }
 
-template <class Robot, bool LDS>
-__global__ __launch_bounds__(kWave) void k_check_poses(const float *__restrict__ scene, int scene_f4,
+template <class Robot>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void k_check_poses(const float *__restrict__ scene, int scene_f4,
                                                        const float *__restrict__ poses, int n,
                                                        uint8_t *__restrict__ out) {
     extern __shared__ float4 lds_scene[];
     CheckCtx ctx;
     ctx.independent = true;
     ctx.key = 0;
-    bind_scene<LDS>(scene, scene_f4, lds_scene, ctx.obs);
+    bind_scene(scene, scene_f4, lds_scene, ctx.obs);
     for (int base = blockIdx.x * kWave; base < n; base += gridDim.x * kWave) {
         const int i = base + threadIdx.x;
         const int src = i < n ? i : n - 1;
@@ -56,15 +56,15 @@ __global__ __launch_bounds__(kWave) void k_check_poses(const float *__restrict__
 
 // One wave per edge (grid-stride over edges).  Pass p of P = ceil(g/64)
 // gives lane l the pose k = l*P + p; pose k is a + (k+1) * ((b-a)/g).
-template <class Robot, bool LDS>
-__global__ __launch_bounds__(kWave) void k_validate_edges(const float *__restrict__ scene, int scene_f4,
+template <class Robot>
+__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void k_validate_edges(const float *__restrict__ scene, int scene_f4,
                                                           const float *__restrict__ edges, int n, int g,
                                                           uint8_t *__restrict__ out) {
     extern __shared__ float4 lds_scene[];
     constexpr int D = Robot::DOF;
     CheckCtx ctx;
     ctx.independent = false;
-    bind_scene<LDS>(scene, scene_f4, lds_scene, ctx.obs);
+    bind_scene(scene, scene_f4, lds_scene, ctx.obs);
     const int lane = threadIdx.x;
     const int passes = (g + kWave - 1) / kWave;
     const float gf = (float)g;
@@ -209,7 +209,7 @@ int num_cus() {
 
 template <class... KArgs, class... Args>
 static void launch_scene_kernel(void (*k)(KArgs...), dim3 grid, size_t scene_f4, hipStream_t st, Args... args) {
-    hipLaunchKernelGGL(k, grid, dim3(kWave), scene_f4 * sizeof(float4), st, args...);
+    hipLaunchKernelGGL(k, grid, dim3(kWave), scene_lds_f4((int)scene_f4) * sizeof(float4), st, args...);
     PRRTC_HIP(hipGetLastError());
 }
 
@@ -217,7 +217,7 @@ template <class Robot>
 static void launch_validate(const float *d_scene, size_t scene_f4, const float *d_edges, int n, int g,
                             uint8_t *d_out, hipStream_t st) {
     const int grid = std::max(1, std::min(n, num_cus() * 16));
-    launch_scene_kernel(k_validate_edges<Robot, true>, dim3(grid), scene_f4, st, d_scene, (int)scene_f4, d_edges,
+    launch_scene_kernel(k_validate_edges<Robot>, dim3(grid), scene_f4, st, d_scene, (int)scene_f4, d_edges,
                         n, g, d_out);
 }
 
@@ -225,7 +225,7 @@ template <class Robot>
 static void launch_check(const float *d_scene, size_t scene_f4, const float *d_poses, int n, uint8_t *d_out,
                          hipStream_t st) {
     const int blocks = std::max(1, std::min((n + kWave - 1) / kWave, num_cus() * 16));
-    launch_scene_kernel(k_check_poses<Robot, true>, dim3(blocks), scene_f4, st, d_scene, (int)scene_f4, d_poses,
+    launch_scene_kernel(k_check_poses<Robot>, dim3(blocks), scene_f4, st, d_scene, (int)scene_f4, d_poses,
                         n, d_out);
 }
 

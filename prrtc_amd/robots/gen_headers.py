@@ -16,7 +16,11 @@ formed only where a check needs them (t_f + R_f * local, constants folded).
 The checks talk to the caller through ``Ctx``:
 
     bool live()                      this lane still needs an answer
-    void env_multi<N>(x, y, z, r, hit)  N spheres vs. the obstacle tables
+    void env_gates<N>(x, y, z, r, hit)  N gate spheres vs. the obstacles
+    bool env_any<N, EARLY>(x, y, z, r, on)  whether one of N leaf spheres hits
+                                     an obstacle (env_any_bounded: with a ball
+                                     that holds them); whole-wave calls.  EARLY:
+                                     leave once every lane has a hit
     bool self(ax, ay, az, bx, by, bz, rsum)   sphere pair (true = hit)
     void hit()                       this lane's pose collides
     void share_gates(uint64_t &)     gate bits after the gate pass (ORed
@@ -267,10 +271,9 @@ def gen_robot_from(m: dict) -> str:
         rs = flit(np.float32(sph[a]["r"]) + np.float32(sph[b]["r"]))
         return f"ctx.self({ca[0]}, {ca[1]}, {ca[2]}, {cb[0]}, {cb[1]}, {cb[2]}, {rs})"
 
-    def env_group(spheres_idx, out, indent, early, bound=None, any_hit=False):
-        """One env_multi call over the spheres; with any_hit only whether some
-        sphere hits is computed (env_any: one running minimum for the group)
-        and `out` uses the bool `eh`, else the per-sphere array eh[]."""
+    def env_group(spheres_idx, call, indent):
+        """The centres and radii of some spheres in arrays ex, ey, ez, er of
+        `n`, and the lines `call` over them."""
         n = len(spheres_idx)
         cs = [centre(i) for i in spheres_idx]
         w(f"{indent}{{")
@@ -278,21 +281,8 @@ def gen_robot_from(m: dict) -> str:
         w(f"{indent}    const float ey[{n}] = {{" + ", ".join(c[1] for c in cs) + "};")
         w(f"{indent}    const float ez[{n}] = {{" + ", ".join(c[2] for c in cs) + "};")
         w(f"{indent}    const float er[{n}] = {{" + ", ".join(flit(sph[i]['r']) for i in spheres_idx) + "};")
-        early_s = "true" if early else "false"
-        fn = "env_any" if any_hit else "env_multi"
-        args = "ex, ey, ez, er" if any_hit else "ex, ey, ez, er, eh"
-        if bound is not None:
-            # the contexts bound only leaf groups (the any-hit form)
-            assert any_hit, "a bound needs the any-hit form"
-            gc, gr = bound
-            fn += "_bounded"
-            args += f", {gc[0]}, {gc[1]}, {gc[2]}, {flit(gr)}"
-        if any_hit:
-            w(f"{indent}    const bool eh = ctx.template {fn}<{n}, {early_s}>({args});")
-        else:
-            w(f"{indent}    bool eh[{n}];")
-            w(f"{indent}    ctx.template {fn}<{n}, {early_s}>({args});")
-        w(f"{indent}    {out}")
+        for line in call:
+            w(f"{indent}    {line}")
         w(f"{indent}}}")
 
     GROUP_MIN_LEAVES = 6
@@ -315,11 +305,13 @@ def gen_robot_from(m: dict) -> str:
 
     env = m["env_checks"]
     w("    uint64_t gate = 0;  /* bit k: env check k's gate sphere hit */")
-    w("    if (ctx.live()) {")
+    w("    if (ctx.any(ctx.live())) {")
     for c0 in range(0, len(env), GATE_CHUNK):
         ks = list(range(c0, min(len(env), c0 + GATE_CHUNK)))
         bits = " | ".join(f"((uint64_t)eh[{j}] << {k})" for j, k in enumerate(ks))
-        env_group([env[k]["gate"] for k in ks], f"gate |= {bits};", "        ", False)
+        env_group([env[k]["gate"] for k in ks],
+                  [f"bool eh[{len(ks)}];", f"ctx.template env_gates<{len(ks)}>(ex, ey, ez, er, eh);",
+                   f"gate |= {bits};"], "        ")
     w("    }")
     # the one point where waves that split the obstacles exchange gate bits:
     # before any early return, so every wave reaches it once per call
@@ -336,9 +328,14 @@ def gen_robot_from(m: dict) -> str:
             continue
         w(f"    /* env leaves: {chk['label']} */")
         w(f"    if (ctx.any(ctx.live() && (gate >> {k} & 1))) {{")
-        w(f"        if (ctx.live() && (gate >> {k} & 1)) {{")
-        env_group(chk["leaves"], "if (eh) ctx.hit();", "            ", True, group_bound(chk), any_hit=True)
-        w("        }")
+        n, bound = len(chk["leaves"]), group_bound(chk)
+        if bound is None:
+            call = f"ctx.template env_any<{n}, true>(ex, ey, ez, er, on)"
+        else:
+            gc, gr = bound
+            call = f"ctx.template env_any_bounded<{n}, true>(ex, ey, ez, er, on, {gc[0]}, {gc[1]}, {gc[2]}, {flit(gr)})"
+        w(f"        const bool on = ctx.live() && (gate >> {k} & 1);")
+        env_group(chk["leaves"], [f"const bool eh = {call};", "if (on && eh) ctx.hit();"], "        ")
         w("        if (ctx.stop()) return;")
         w("    }")
     # self groups are numbered in emission order; ctx.mine(j) lets a

@@ -1,0 +1,98 @@
+"""The broad phase lists the obstacles a wave's poses can touch, 64 at a time
+and dealt to the waves that share a pass.  Verdicts at the sizes where a list
+can go wrong -- one obstacle, the ends of a 64-obstacle block in each table,
+full tables -- against the oracle; a pose that is no number; and the ball
+itself (on the CPU): nothing out of its reach can collide."""
+import numpy as np
+import pytest
+
+from conftest import NEAR, edge_margins
+
+F32 = np.float32
+# spheres, capsules, z-capsules, cuboids, z-cuboids
+COUNTS = [(1, 0, 0, 0, 0), (0, 0, 0, 1, 0), (63, 1, 0, 0, 0), (64, 0, 1, 0, 0), (0, 65, 0, 0, 0), (0, 0, 64, 0, 1),
+          (20, 20, 20, 20, 20), (0, 0, 0, 63, 2), (0, 0, 0, 0, 129), (4096, 0, 0, 0, 0), (0, 2048, 0, 0, 0),
+          (0, 0, 0, 0, 1024)]
+
+
+def _scene(counts, seed):
+    """Small obstacles through the workspace, off the base axis."""
+    from prrtc_amd import scenes as S
+    rng = np.random.default_rng(seed)
+    size = 0.12 / max(1.0, sum(counts) / 24.0) ** (1 / 3)   # about the same share of the space in obstacles
+
+    def centre():
+        while True:
+            c = rng.uniform([-0.9, -0.9, 0.0], [0.9, 0.9, 1.3])
+            if np.hypot(c[0], c[1]) > 0.35:
+                return c
+    sph = [S.sphere(centre(), size) for _ in range(counts[0])]
+    cap = [S.cylinder_center(centre(), rng.uniform(-3, 3, 3), size / 2, 2 * size) for _ in range(counts[1])]
+    zcap = [S.cylinder_center(centre(), (0, 0, 0), size / 2, 2 * size) for _ in range(counts[2])]
+    cub = [S.cuboid(centre(), rng.uniform(-3, 3, 3), rng.uniform(size / 2, size, 3)) for _ in range(counts[3])]
+    zcub = [S.cuboid(centre(), (0, 0, rng.uniform(-3, 3)), rng.uniform(size / 2, size, 3)) for _ in range(counts[4])]
+    return S.Scene.build(sph, cap, zcap, cub, zcub)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("robot", ["panda", "fetch", "baxter"])
+@pytest.mark.parametrize("counts", COUNTS, ids=str)
+def test_edges_against_oracle(robot, counts, gpu, oracle_robots):
+    from prrtc_amd.robots import limits
+    R = oracle_robots[robot]
+    sc = _scene(counts, 5 + sum(counts))
+    lo, span = limits(robot)
+    rng = np.random.default_rng(11)
+    n = 200 if sum(counts) < 1000 else 60
+    a = (lo + span * rng.random((n, len(lo)), dtype=F32)).astype(F32)
+    b = np.clip(a + rng.normal(size=a.shape) * rng.choice([0.01, 0.2], (n, 1)), lo, lo + span).astype(F32)
+    edges = np.stack([a, b], 1)
+    got = gpu.validate_edges(robot, sc, edges, 32)
+    want = R.validate_edges(sc, edges, 32)
+    flips = np.nonzero(got != want)[0]
+    assert np.all(edge_margins(R, sc, edges[flips], 32) < NEAR)
+
+
+@pytest.mark.gpu
+def test_pose_that_is_no_number(gpu, oracle_robots):
+    """A cuboid's test takes a NaN position for a hit (utils.cuh:158-175: the
+    NaN is dropped by max(0, .)), a sphere's for none; neither may be lost
+    because the wave's ball has no radius."""
+    import torch
+    from prrtc_amd import scenes as S
+    far = (3.0, 3.0, 3.0)
+    a = np.tile(np.array([0, -0.8, 0, -2.0, 0, 1.6, 0.8], F32), (3, 1))
+    b = a + F32(0.1)
+    b[1, 0] = np.nan      # every pose
+    edges = torch.from_numpy(np.stack([a, b], 1)).cuda()
+    for sc, want in ((S.Scene.build(cuboids=[S.cuboid(far, (0, 0, 0), (0.1,) * 3)]), [1, 0, 1]),
+                     (S.Scene.build(spheres=[S.sphere(far, 0.1)]), [1, 1, 1])):
+        packed = torch.from_numpy(gpu.pack_scene(sc)).cuda()
+        out = torch.full((3,), 7, dtype=torch.uint8, device="cuda")
+        gpu.validate_edges_async("panda", packed.data_ptr(), packed.numel(), edges.data_ptr(), 3, 32, out.data_ptr())
+        torch.cuda.synchronize()
+        assert out.cpu().tolist() == want
+
+
+def test_nothing_out_of_reach_collides():
+    """The ball in float32: midpoint of the first and last point, radius
+    sqrt(max d2) (1 + 2^-16), obstacle ball padded by 2^-16 and 1 mm.  An
+    obstacle ball just out of reach leaves every exact sphere test positive."""
+    rng = np.random.default_rng(3)
+    worst = np.inf
+    for _ in range(4000):
+        scale = 10 ** rng.uniform(-3, 3)
+        p = (rng.normal(size=(64, 3)) * scale * 10 ** rng.uniform(-4, 0) + rng.normal(size=3) * scale).astype(F32)
+        r, ro = F32(10 ** rng.uniform(-3, 0)), F32(10 ** rng.uniform(-3, 0) * scale)
+        c = F32(0.5) * (p[0] + p[-1])
+        radius = np.sqrt(np.max(np.sum((p - c) ** 2, 1, dtype=F32))) * F32(1 + 2.0 ** -16)
+        rb = F32(radius + r) + F32(ro * F32(1 + 2.0 ** -16) + F32(1e-3))
+        # an obstacle just out of reach, in the direction of the farthest point
+        u = (p[np.argmax(np.sum((p - c) ** 2, 1))] - c).astype(np.float64)
+        u = u / max(np.linalg.norm(u), 1e-30) if np.any(u) else np.array([1.0, 0, 0])
+        o = (c + u * (float(rb) * (1 + rng.uniform(0, 1e-6)))).astype(F32)
+        if not np.sum((o - c) ** 2, dtype=F32) > F32(rb * rb):
+            continue   # in reach: tested exactly
+        value = np.sum((o - p) ** 2, 1, dtype=F32) - F32(ro + r) ** 2
+        worst = min(worst, float(value.min()))
+    assert worst > 0
