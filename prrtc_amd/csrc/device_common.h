@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "robots/baxter.gen.h"
 #include "robots/fetch.gen.h"
 #include "robots/panda.gen.h"
@@ -289,75 +291,59 @@ __device__ __forceinline__ float z_cuboid_test(const float4 &c, const float4 &a1
 // Smallest test value of obstacle i (wave-uniform) against N spheres per
 // lane, lowered into m[n] (ANY: into m[0], for callers that want only
 // whether some sphere hits).  A NaN test value is dropped by fminf as it
-// would fail `< 0`.  With CULL each sphere first asks whether any lane is
-// within reach of the obstacle's ball: of the N spheres of a link near an
-// obstacle most are not, and the exact test costs three times as much.
-template <int N, bool LOCAL, bool ANY, bool CULL>
+// would fail `< 0`.  far(n, ball) says (wave-uniformly) that sphere n is out
+// of the obstacle's reach on every lane; the obstacle's rows are read once
+// for all N.  ASK_ALL: asking costs no vector instruction, so it is asked for
+// spheres and z-capsules too, whose tests are as cheap as a cull.
+template <int N, bool LOCAL, bool ANY, bool ASK_ALL, class Far>
 __device__ __forceinline__ void test_obstacle(const Obstacles &o, int i, const float *x, const float *y,
-                                              const float *z, const float *r, float *m) {
+                                              const float *z, const float *r, float *m, Far far) {
 #pragma clang fp contract(off)
+    auto each = [&](auto cheap, auto test) {
+#pragma unroll
+        for (int n = 0; n < N; n++) {
+            if ((ASK_ALL || !cheap.value) && far(n)) continue;
+            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], test(x[n], y[n], z[n], r[n]));
+        }
+    };
     if (i < o.n_sph) {
         const float4 s = ld_obs<LOCAL>(o.sph + i);
-#pragma unroll
-        for (int n = 0; n < N; n++) m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], sphere_test(s, x[n], y[n], z[n], r[n]));
+        each(std::true_type{}, [&](float a, float b, float c, float d) { return sphere_test(s, a, b, c, d); });
         return;
     }
     i -= o.n_sph;
-    float4 b;
-    if constexpr (CULL) b = ld_obs<LOCAL>(o.ball + i);
-    auto far = [&](int n) {
-#pragma clang fp contract(off)
-        if constexpr (CULL) {
-            const float rb = r[n] + b.w;
-            return ballot(!(sq3(x[n] - b.x, y[n] - b.y, z[n] - b.z) > rb * rb)) == 0;
-        } else {
-            return false;
-        }
-    };
     if (i < o.n_cap) {
         const float4 p = ld_obs<LOCAL>(o.cap + 2 * i), v = ld_obs<LOCAL>(o.cap + 2 * i + 1);
-#pragma unroll
-        for (int n = 0; n < N; n++) {
-            if (far(n)) continue;
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], capsule_test(p, v, x[n], y[n], z[n], r[n]));
-        }
+        each(std::false_type{}, [&](float a, float b, float c, float d) { return capsule_test(p, v, a, b, c, d); });
         return;
     }
     i -= o.n_cap;
     if (i < o.n_zcap) {
         const float4 p = ld_obs<LOCAL>(o.zcap + 2 * i), v = ld_obs<LOCAL>(o.zcap + 2 * i + 1);
-#pragma unroll
-        for (int n = 0; n < N; n++)
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], z_capsule_test(p, v, x[n], y[n], z[n], r[n]));
+        each(std::true_type{}, [&](float a, float b, float c, float d) { return z_capsule_test(p, v, a, b, c, d); });
         return;
     }
     i -= o.n_zcap;
     if (i < o.n_cub) {
-        const float4 c = ld_obs<LOCAL>(o.cub + 4 * i), a1 = ld_obs<LOCAL>(o.cub + 4 * i + 1),
+        const float4 p = ld_obs<LOCAL>(o.cub + 4 * i), a1 = ld_obs<LOCAL>(o.cub + 4 * i + 1),
                      a2 = ld_obs<LOCAL>(o.cub + 4 * i + 2), a3 = ld_obs<LOCAL>(o.cub + 4 * i + 3);
-#pragma unroll
-        for (int n = 0; n < N; n++) {
-            if (far(n)) continue;
-            m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], cuboid_test(c, a1, a2, a3, x[n], y[n], z[n], r[n]));
-        }
+        each(std::false_type{}, [&](float a, float b, float c, float d) { return cuboid_test(p, a1, a2, a3, a, b, c, d); });
         return;
     }
     i -= o.n_cub;
-    const float4 c = ld_obs<LOCAL>(o.zcub + 4 * i), a1 = ld_obs<LOCAL>(o.zcub + 4 * i + 1),
+    const float4 p = ld_obs<LOCAL>(o.zcub + 4 * i), a1 = ld_obs<LOCAL>(o.zcub + 4 * i + 1),
                  a2 = ld_obs<LOCAL>(o.zcub + 4 * i + 2);
-#pragma unroll
-    for (int n = 0; n < N; n++) {
-        if (far(n)) continue;
-        m[ANY ? 0 : n] = fminf(m[ANY ? 0 : n], z_cuboid_test(c, a1, a2, x[n], y[n], z[n], r[n]));
-    }
+    each(std::false_type{}, [&](float a, float b, float c, float d) { return z_cuboid_test(p, a1, a2, a, b, c, d); });
 }
 
 // sphere_environment_in_collision (utils.cuh:211-242) for N spheres per
 // lane, whose answer is wanted sphere by sphere: hit[n] on each live lane.
-// All 64 lanes call it; `on` marks the live ones (at least one).
+// All 64 lanes call it; `on` marks the live ones (at least one).  The ball of
+// sphere n's positions is left on lane k0 + n of `balls`.
 template <int N, bool LOCAL>
 __device__ __forceinline__ void env_hits(const Obstacles &o, Share sh, const float (&x)[N], const float (&y)[N],
-                                         const float (&z)[N], const float (&r)[N], bool on, bool (&hit)[N]) {
+                                         const float (&z)[N], const float (&r)[N], bool on, bool (&hit)[N],
+                                         int k0, WaveBall &balls) {
 #pragma clang fp contract(off)
     const uint64_t live = ballot(on);
     const int lane = threadIdx.x & (kWave - 1);
@@ -365,24 +351,32 @@ __device__ __forceinline__ void env_hits(const Obstacles &o, Share sh, const flo
     float m[N];
 #pragma unroll
     for (int n = 0; n < N; n++) m[n] = __builtin_huge_valf();
-    for (int base = 0; base < mine; base += kWave) {
+    int base = 0;
+    do {   // at least once: the balls are wanted in an empty scene too
         const int j = base + lane;
         const bool have = j < mine;
-        const float4 b = obstacle_ball<LOCAL>(o, have ? (j << sh.shift) + sh.part : 0);
+        float4 b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (mine > 0) b = obstacle_ball<LOCAL>(o, have ? (j << sh.shift) + sh.part : 0);
         uint64_t near[N];
 #pragma unroll
         for (int n = 0; n < N; n++) {
             const WaveBall c = wave_ball(x[n], y[n], z[n], on, live);
             near[n] = ballot(have && in_reach(b, c, c.r + r[n]));
+            int ln = lane;
+            asm volatile("" : "+v"(ln));   // compared here: kept across the edge loop, a mask per gate spills SGPRs
+            if (ln == k0 + n) balls = c;
         }
+        // obstacle by obstacle, each against the spheres that list it
+        uint64_t w = 0;
 #pragma unroll
-        for (int n = 0; n < N; n++) {
-            for (uint64_t w = near[n]; w; w &= w - 1) {
-                const int i = __builtin_amdgcn_readfirstlane(((base + __builtin_ctzll(w)) << sh.shift) + sh.part);
-                test_obstacle<1, LOCAL, false, false>(o, i, x + n, y + n, z + n, r + n, m + n);
-            }
+        for (int n = 0; n < N; n++) w |= near[n];
+        for (; w; w &= w - 1) {
+            const int bit = __builtin_ctzll(w);
+            const int i = __builtin_amdgcn_readfirstlane(((base + bit) << sh.shift) + sh.part);
+            test_obstacle<N, LOCAL, false, true>(o, i, x, y, z, r, m, [&](int n) { return !((near[n] >> bit) & 1); });
         }
-    }
+        base += kWave;
+    } while (base < mine);
 #pragma unroll
     for (int n = 0; n < N; n++) hit[n] = m[n] < 0.0f;
 }
@@ -405,7 +399,13 @@ __device__ __forceinline__ bool env_group(const Obstacles &o, Share sh, const fl
         const float4 b = obstacle_ball<LOCAL>(o, have ? (j << sh.shift) + sh.part : 0);
         for (uint64_t w = ballot(have && in_reach(b, c, reach)); w; w &= w - 1) {
             const int i = __builtin_amdgcn_readfirstlane(((base + __builtin_ctzll(w)) << sh.shift) + sh.part);
-            test_obstacle<N, LOCAL, true, true>(o, i, x, y, z, r, m);
+            // of a link's spheres near an obstacle most are out of its reach
+            // on every lane; the exact test costs three times this one
+            const float4 ob = obstacle_ball<LOCAL>(o, i);
+            test_obstacle<N, LOCAL, true, false>(o, i, x, y, z, r, m, [&](int n) {
+                const float rb = r[n] + ob.w;
+                return ballot(!(sq3(x[n] - ob.x, y[n] - ob.y, z[n] - ob.z) > rb * rb)) == 0;
+            });
             if (EARLY && ballot(on && !(m[0] < 0.0f)) == 0) return true;
         }
     }
@@ -450,6 +450,53 @@ __device__ __forceinline__ bool self_hit(float ax, float ay, float az, float bx,
     return fmaf(-rs, rs, sq3(ax - bx, ay - by, az - bz)) < 0.0f;
 }
 
+// Self-collision groups by the same balls.  A group is a pair of gate spheres
+// (a link's each); `pairs` packs one group per word: the gates' numbers and
+// the sum of their radii, padded and rounded up to binary16 by the
+// generator.  With the ball of gate k's positions on lane k, every lane takes
+// one group: when the two balls stay apart by more than the radii, no live
+// lane's gates touch and the group needs no test at all.  (A gate test costs
+// some 30 instructions and a branch, and Baxter has 355; here 64 groups cost
+// as much as one.  30k Baxter edges 542 -> 284 us, an uneven batch of 128
+// problems 219 -> 163 ms, a served burst 105 -> 63 ms.)  near[w] gets the
+// groups 64 w .. 64 w + 63 that do, of those whose number is sh.part mod
+// 2^sh.shift (the wave's own).
+constexpr int kSelfWords = 6;   // up to 384 groups
+
+template <int NS>
+__device__ __forceinline__ void self_groups_own(Share sh, uint64_t (&near)[kSelfWords]) {
+    static_assert(NS <= 64 * kSelfWords, "groups fit the mask");
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint64_t own = ballot((lane & ((1 << sh.shift) - 1)) == sh.part);   // 64 is a multiple of 2^shift
+#pragma unroll
+    for (int w = 0; w < (NS + 63) / 64; w++) near[w] = own;
+}
+
+template <int NS>
+__device__ __forceinline__ void self_groups_near(Share sh, const uint32_t *pairs, const WaveBall &balls,
+                                                 uint64_t (&near)[kSelfWords]) {
+#pragma clang fp contract(off)
+    static_assert(NS <= 64 * kSelfWords, "groups fit the mask");
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool own = (lane & ((1 << sh.shift) - 1)) == sh.part;
+    auto from = [](float v, uint32_t k) {
+        return __int_as_float(__builtin_amdgcn_ds_bpermute((int)(k << 2), __float_as_int(v)));
+    };
+    uint32_t p[(NS + 63) / 64];
+#pragma unroll
+    for (int w = 0; w < (NS + 63) / 64; w++) p[w] = pairs[64 * w + lane < NS ? 64 * w + lane : NS - 1];
+#pragma unroll
+    for (int w = 0; w < (NS + 63) / 64; w++) {
+#pragma clang fp contract(off)
+        const uint32_t a = p[w] & 0xff, b = (p[w] >> 8) & 0xff;
+        const float dx = from(balls.x, a) - from(balls.x, b), dy = from(balls.y, a) - from(balls.y, b),
+                    dz = from(balls.z, a) - from(balls.z, b);
+        const uint16_t h = (uint16_t)(p[w] >> 16);
+        const float reach = (from(balls.r, a) + from(balls.r, b)) + (float)__builtin_bit_cast(_Float16, h);
+        near[w] = ballot(own && 64 * w + lane < NS && !(sq3(dx, dy, dz) > reach * reach));
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Check context driven by the generated robot code, for a pass of up to 64
 // poses (one per lane).
@@ -468,18 +515,34 @@ struct CheckCtx {
     bool dead;
     bool independent;
     int key;
+    WaveBall balls;                   // lane k: the ball of gate k's positions
+    uint64_t near[kSelfWords];        // self-collision groups to test
 
     __device__ __forceinline__ bool live() const { return !coll && !dead; }
     __device__ __forceinline__ bool any(bool p) const { return ballot(p) != 0; }
     // Self-collision group j (numbered in check order) is this wave's to
-    // test; a lone wave tests every group.
-    __device__ __forceinline__ bool mine(int) const { return true; }
-    // N gate spheres against the obstacles, hit[n] on each live lane; called
-    // by the whole wave while some lane is live.
+    // test: its own, and not ruled out by the gates' balls.
+    __device__ __forceinline__ bool mine(int j) const { return (near[j >> 6] >> (j & 63)) & 1; }
+    // Any of the groups j .. j + n - 1 (of one 64-group word).
+    __device__ __forceinline__ bool mine_any(int j, int n) const {
+        return ((near[j >> 6] >> (j & 63)) & ((1ull << n) - 1)) != 0;
+    }
+    template <int NS>
+    __device__ __forceinline__ void self_own() { self_groups_own<NS>(Share{}, near); }
+    template <int NS>
+    __device__ __forceinline__ void self_near(const uint32_t *pairs) {
+        self_groups_near<NS>(Share{}, pairs, balls, near);
+    }
+    // The ball of a gate that never moves, at number k.
+    __device__ __forceinline__ void fixed_gate(int k, float x, float y, float z) {
+        if ((int)(threadIdx.x & (kWave - 1)) == k) balls = WaveBall{x, y, z, 0.0f};
+    }
+    // Gate spheres k0 .. k0 + N - 1 against the obstacles, hit[n] on each
+    // live lane; called by the whole wave while some lane is live.
     template <int N>
-    __device__ __forceinline__ void env_gates(const float (&x)[N], const float (&y)[N], const float (&z)[N],
-                                              const float (&r)[N], bool (&hit)[N]) const {
-        env_hits<N, false>(obs, Share{}, x, y, z, r, live(), hit);
+    __device__ __forceinline__ void env_gates(int k0, const float (&x)[N], const float (&y)[N], const float (&z)[N],
+                                              const float (&r)[N], bool (&hit)[N]) {
+        env_hits<N, false>(obs, Share{}, x, y, z, r, live(), hit, k0, balls);
     }
     // Whether any of the N spheres of a leaf group hits an obstacle, on the
     // lanes with `on` (at least one); called by the whole wave.
@@ -530,7 +593,7 @@ struct SphereRobot {     // Robots.hh:190-237; fkcc<Sphere>, utils.cuh:330-334
         const float x[1] = {q[0]}, y[1] = {q[1]}, z[1] = {q[2]}, r[1] = {1.0f};
         bool h[1];
         if (ctx.any(ctx.live())) {
-            ctx.template env_gates<1>(x, y, z, r, h);
+            ctx.template env_gates<1>(0, x, y, z, r, h);
             if (ctx.live() && h[0]) ctx.hit();
         }
         ctx.stop();

@@ -74,7 +74,6 @@ struct TaskCtx : CheckCtx {
     Share share;
     bool shared_stop; // the task runs on several waves: stop keys go through LDS
     bool wide_ok;     // its chain passes may give each wave poses of its own
-    unsigned mine12;  // bit i: self groups j with j mod 12 == i are this wave's (12 = lcm of 1..4)
     __device__ __forceinline__ void share_gates(uint64_t &gate) {
         const int W = waves;
         if (W == 1) return;
@@ -86,13 +85,17 @@ struct TaskCtx : CheckCtx {
         __syncthreads();   // gbuf is written again by the next pass
         gate = g;
     }
-    static_assert(kMaxTaskWaves <= 4, "the 12-group pattern of mine12 needs 12 % waves == 0");
-    __device__ __forceinline__ bool mine(int j) const { return (mine12 >> (j % 12)) & 1u; }
+    template <int NS>
+    __device__ __forceinline__ void self_own() { self_groups_own<NS>(share, near); }
+    template <int NS>
+    __device__ __forceinline__ void self_near(const uint32_t *pairs) {
+        self_groups_near<NS>(share, pairs, balls, near);
+    }
     // The obstacle tables of a task are always staged in LDS.
     template <int N>
-    __device__ __forceinline__ void env_gates(const float (&x)[N], const float (&y)[N], const float (&z)[N],
-                                              const float (&r)[N], bool (&hit)[N]) const {
-        env_hits<N, true>(obs, share, x, y, z, r, live(), hit);
+    __device__ __forceinline__ void env_gates(int k0, const float (&x)[N], const float (&y)[N], const float (&z)[N],
+                                              const float (&r)[N], bool (&hit)[N]) {
+        env_hits<N, true>(obs, share, x, y, z, r, live(), hit, k0, balls);
     }
     template <int N, bool EARLY>
     __device__ __forceinline__ bool env_any(const float (&x)[N], const float (&y)[N], const float (&z)[N],
@@ -169,10 +172,6 @@ __device__ __attribute__((always_inline)) void plan_task(const PlanDesc &d, Plan
         ctx.share.shift = gs == 4 ? 2 : gs == 2 ? 1 : 0;
         ctx.waves = gs;
         ctx.gbase = gw * gs;
-        unsigned m = 0;
-        for (int i = 0; i < 12; i++) m |= (unsigned)(i % gs == wi) << i;
-        // uniform over the wave: the group branches stay scalar branches
-        ctx.mine12 = (unsigned)__builtin_amdgcn_readfirstlane((int)m);
     };
     const bool wide_ok = __builtin_amdgcn_readfirstlane((int)ctx_in.wide_ok) != 0 && d.wide_from >= 0;
     // pose groups for n poses: one pass where the waves allow it

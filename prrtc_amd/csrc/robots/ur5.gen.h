@@ -130,7 +130,7 @@ __device__ __forceinline__ void check(const float *q, Ctx &ctx) {
             const float ez[7] = {0.08915899693965912f, 0.08915899693965912f + -0.24285714328289032f * R1_21, -0.19870834052562714f * R2_21 + t2_2, t3_2, 0.02500000037252903f * M4_22 + t3_2, 0.02500000037252903f * R4_21 + t5_2, 2.449293581093244e-18f * R5_20 + 0.12229999899864197f * R4_21 + t5_2};
             const float er[7] = {0.10999999940395355f, 0.3080083429813385f, 0.2487083375453949f, 0.07000000029802322f, 0.07000000029802322f, 0.06499999761581421f, 0.03999999910593033f};
             bool eh[7];
-            ctx.template env_gates<7>(ex, ey, ez, er, eh);
+            ctx.template env_gates<7>(0, ex, ey, ez, er, eh);
             gate |= ((uint64_t)eh[0] << 0) | ((uint64_t)eh[1] << 1) | ((uint64_t)eh[2] << 2) | ((uint64_t)eh[3] << 3) | ((uint64_t)eh[4] << 4) | ((uint64_t)eh[5] << 5) | ((uint64_t)eh[6] << 6);
         }
     }
@@ -215,6 +215,7 @@ __device__ __forceinline__ void check(const float *q, Ctx &ctx) {
         }
         if (ctx.stop()) return;
     }
+    ctx.template self_own<33>();
     /* self: wrist_2_link vs. base_link */
     if (ctx.mine(0)) {
         const bool g = ctx.live() && ctx.self(t4_0, t4_1, t3_2, 0.0f, 0.0f, 0.04500000178813934f, 0.13500000536441803f);

@@ -56,6 +56,14 @@ def flit(v: float) -> str:
     return r + "f"
 
 
+def half_up(v: float) -> int:
+    """Bits of the smallest binary16 at or above v (v > 0)."""
+    h = np.float16(v)
+    if float(h) < v:
+        h = np.nextafter(h, np.float16(np.inf))
+    return int(h.view(np.uint16))
+
+
 class Lin:
     """A linear form sum(c_i * var_i) + const, with constant folding."""
 
@@ -262,6 +270,12 @@ def gen_robot_from(m: dict) -> str:
     # the self-collision gate pairs and their sphere pairs.  The verdict is
     # the same OR of gated terms the reference evaluates (utils.cuh:336-5270).
     GATE_CHUNK = 12
+    def pair_reach(chk):
+        """Distance beyond which a self group's gates cannot touch: the sum of
+        their radii, padded by 2^-16 relative and 1 mm absolute."""
+        a, b = chk["gate"]
+        return (float(sph[a]["r"]) + float(sph[b]["r"])) * (1.0 + 2.0 ** -16) + 1e-3
+
     w("template <class Ctx>")
     w("__device__ __forceinline__ void check(const float *q, Ctx &ctx) {")
     w("    PRRTC_FK_BODY")
@@ -310,7 +324,7 @@ def gen_robot_from(m: dict) -> str:
         ks = list(range(c0, min(len(env), c0 + GATE_CHUNK)))
         bits = " | ".join(f"((uint64_t)eh[{j}] << {k})" for j, k in enumerate(ks))
         env_group([env[k]["gate"] for k in ks],
-                  [f"bool eh[{len(ks)}];", f"ctx.template env_gates<{len(ks)}>(ex, ey, ez, er, eh);",
+                  [f"bool eh[{len(ks)}];", f"ctx.template env_gates<{len(ks)}>({c0}, ex, ey, ez, er, eh);",
                    f"gate |= {bits};"], "        ")
     w("    }")
     # the one point where waves that split the obstacles exchange gate bits:
@@ -338,10 +352,34 @@ def gen_robot_from(m: dict) -> str:
         env_group(chk["leaves"], [f"const bool eh = {call};", "if (on && eh) ctx.hit();"], "        ")
         w("        if (ctx.stop()) return;")
         w("    }")
-    # self groups are numbered in emission order; ctx.mine(j) lets a
-    # context whose waves share a pose set give each group to one wave
-    for j, (kind, k) in enumerate([o for o in m["order"] if o[0] == "self"]):
-        chk = m["self_checks"][k]
+    # Self groups are numbered in emission order; ctx.mine(j) lets a context
+    # whose waves share a pose set give each group to one wave, and rules out
+    # the groups whose gates stay apart over the whole wave (by the balls of
+    # the gate pass, where every moving gate of the self groups took part in
+    # it: forming a ball costs about as much as a group's own gate test).
+    selfs = [m["self_checks"][k] for kind, k in m["order"] if kind == "self"]
+    number = {c["gate"]: k for k, c in enumerate(env)}
+    extra = [g for g in sorted({g for c in selfs for g in c["gate"]}) if g not in number]
+    by_balls = bool(selfs) and all(sph[g]["frame"] < 0 for g in extra) and len(env) + len(extra) <= 64
+    if by_balls:
+        for g in extra:
+            number[g] = len(number)
+            c = centre(g)
+            w(f"    ctx.fixed_gate({number[g]}, {c[0]}, {c[1]}, {c[2]});")
+        w(f"    ctx.template self_near<{len(selfs)}>(self_gates);")
+        words = [number[c["gate"][0]] | number[c["gate"][1]] << 8 | half_up(pair_reach(c)) << 16 for c in selfs]
+        at = next(i for i, line in enumerate(L) if line == "template <class Ctx>")
+        L[at:at] = ["// self groups: the two gates' numbers and, rounded up to binary16, their reach",
+                    f"__device__ const uint32_t self_gates[{len(words)}] = {{" +
+                    ", ".join(f"{x:#x}u" for x in words) + "};", ""]
+    elif selfs:
+        w(f"    ctx.template self_own<{len(selfs)}>();")
+    BLOCK = 16   # groups passed over together where there are many (blocks do not cross a 64-group word)
+    for j, chk in enumerate(selfs):
+        if len(selfs) > 64 and j % BLOCK == 0:
+            if j:
+                w("    }")
+            w(f"    if (ctx.mine_any({j}, {min(BLOCK, len(selfs) - j)})) {{")
         ga, gb = chk["gate"]
         w(f"    /* self: {chk['label']} */")
         w(f"    if (ctx.mine({j})) {{")
@@ -367,6 +405,8 @@ def gen_robot_from(m: dict) -> str:
             w("            }")
         w("            if (ctx.stop()) return;")
         w("        }")
+        w("    }")
+    if len(selfs) > 64:
         w("    }")
     w("}")
     w("#undef PRRTC_FK_BODY")

@@ -96,3 +96,31 @@ def test_nothing_out_of_reach_collides():
         value = np.sum((o - p) ** 2, 1, dtype=F32) - F32(ro + r) ** 2
         worst = min(worst, float(value.min()))
     assert worst > 0
+
+
+@pytest.mark.parametrize("robot", ["panda", "fetch", "baxter"])
+def test_self_group_words(robot):
+    """Each self group's word names its two gates by the number of their ball
+    and holds at least the sum of their radii (padded by 1 mm, rounded up)."""
+    import os
+    import re
+    from prrtc_amd.robots import load_model
+    m = load_model(robot)
+    here = os.path.join(os.path.dirname(__file__), "..", "prrtc_amd", "csrc", "robots")
+    text = open(os.path.join(here, robot + ".gen.h")).read()
+    words = [int(w, 16) for w in re.findall(r"0x[0-9a-f]+", re.search(r"self_gates\[\d+\] = \{(.*)\}", text).group(1))]
+    selfs = [m["self_checks"][k] for kind, k in m["order"] if kind == "self"]
+    number = [c["gate"] for c in m["env_checks"]]
+    # gates that never move follow the environment gates, by their fixed_gate lines
+    for k, xyz in re.findall(r"ctx\.fixed_gate\((\d+), (.*)\);", text):
+        at = [np.float32(v.strip(" f")) for v in xyz.split(",")]
+        number.append(next(i for i, s in enumerate(m["spheres"])
+                           if s["frame"] < 0 and np.allclose(s["local"], at, atol=1e-7)))
+        assert int(k) == len(number) - 1
+    assert len(words) == len(selfs) and len(number) <= 64
+    for w, chk in zip(words, selfs):
+        a, b = chk["gate"]
+        assert (number[w & 0xff], number[w >> 8 & 0xff]) == (a, b)
+        reach = float(np.array(w >> 16, np.uint16).view(np.float16))
+        rs = m["spheres"][a]["r"] + m["spheres"][b]["r"]
+        assert rs + 0.99e-3 <= reach <= (rs + 1e-3) * 1.002
