@@ -562,6 +562,11 @@ struct CheckCtx {
     __device__ __forceinline__ bool self(float ax, float ay, float az, float bx, float by, float bz, float rs) const {
         return self_hit(ax, ay, az, bx, by, bz, rs);
     }
+    __device__ __forceinline__ bool near_point(float ax, float ay, float az, float bx, float by, float bz,
+                                               float d2) const {
+#pragma clang fp contract(off)
+        return !(sq3(ax - bx, ay - by, az - bz) > d2);
+    }
     __device__ __forceinline__ void hit() { coll = true; }
     // Gate bits of this lane's pose after the gate pass.  A context whose
     // waves split the obstacle tables ORs them across its waves; here every

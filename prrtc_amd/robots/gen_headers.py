@@ -22,6 +22,7 @@ The checks talk to the caller through ``Ctx``:
                                      that holds them); whole-wave calls.  EARLY:
                                      leave once every lane has a hit
     bool self(ax, ay, az, bx, by, bz, rsum)   sphere pair (true = hit)
+    bool near_point(ax, ay, az, bx, by, bz, d2)  within sqrt(d2) (NaN: yes)
     void hit()                       this lane's pose collides
     void share_gates(uint64_t &)     gate bits after the gate pass (ORed
                                      across waves that split the obstacles)
@@ -276,6 +277,43 @@ def gen_robot_from(m: dict) -> str:
         a, b = chk["gate"]
         return (float(sph[a]["r"]) + float(sph[b]["r"])) * (1.0 + 2.0 ** -16) + 1e-3
 
+    # Panda's forearm-hand group (216 pairs) and its like were 2,000 of the
+    # 4,900 VALU instructions of a free pass: 1M edges 7.9 -> 6.7 ms, 64 edges
+    # 24.9 -> 21.6 us, one solve 204 -> 195 us.  Splitting smaller groups too
+    # left Panda as it was and cost Fetch's edge kernel 4% (72 -> 75 us).
+    SPLIT_MIN_PAIRS = 48
+
+    def split_pairs(chk):
+        """(outer spheres, inner spheres, inner gate, radius R) of a self group
+        whose pairs are all of outer x inner, with the inner spheres in the
+        ball of radius R about their gate; None where a group's pairs are
+        cheaper tested outright.  An outer sphere's test against the ball
+        costs about 10 instructions with its branch, a pair 8.  Of the two
+        links the one expected to cost less is the outer: with the gates in
+        touch, an outer sphere is taken to be within reach of the ball with
+        the ratio of the two reaches' volumes."""
+        best = None
+        if len(chk["pairs"]) < SPLIT_MIN_PAIRS:
+            return None
+        for side in (0, 1):
+            outer, inner = [], []
+            for p in chk["pairs"]:
+                if p[side] not in outer:
+                    outer.append(p[side])
+                if p[1 - side] not in inner:
+                    inner.append(p[1 - side])
+            gate = chk["gate"][1 - side]
+            n = len(outer) * len(inner)
+            if n != len(chk["pairs"]) or len(inner) < 5 or any(sph[x]["frame"] != sph[gate]["frame"] for x in inner):
+                continue
+            R = ball_of(gate, inner)
+            gates = sum(float(sph[x]["r"]) for x in chk["gate"])
+            near = sum(min(1.0, ((R + float(sph[x]["r"])) / gates) ** 3) for x in outer) / len(outer)
+            cost = 10 * len(outer) + 8 * n * near
+            if cost < 8 * n and (best is None or cost < best[0]):
+                best = (cost, (outer, inner, gate, R))
+        return best and best[1]
+
     w("template <class Ctx>")
     w("__device__ __forceinline__ void check(const float *q, Ctx &ctx) {")
     w("    PRRTC_FK_BODY")
@@ -299,23 +337,27 @@ def gen_robot_from(m: dict) -> str:
             w(f"{indent}    {line}")
         w(f"{indent}}}")
 
+    def ball_of(gate, spheres):
+        """Radius of the ball about a gate's centre that holds spheres riding
+        on its frame: max |local - local_gate| + r, padded by 2^-16 relative
+        and 1 mm absolute, rounded up to float32."""
+        R = max(float(np.linalg.norm(np.array(sph[x]["local"], dtype=np.float64) -
+                                     np.array(sph[gate]["local"], dtype=np.float64))) + float(sph[x]["r"])
+                for x in spheres)
+        return float(np.nextafter(np.float32(R * (1.0 + 2.0 ** -16) + 1e-3), np.float32(np.inf)))
+
     GROUP_MIN_LEAVES = 6
 
     def group_bound(chk):
-        """Ball about the gate centre that holds every leaf sphere of the
-        check, when the leaves ride on the gate's frame (rigidly): radius
-        max |local_leaf - local_gate| + r_leaf, padded by 2^-16 relative and
-        1 mm absolute, rounded up to float32.  None when a leaf is on another
-        frame, or when the check has fewer than GROUP_MIN_LEAVES leaves."""
+        """Ball about the gate centre (ball_of) that holds every leaf sphere
+        of the check, when the leaves ride on the gate's frame (rigidly).
+        None when a leaf is on another frame, or when the check has fewer than
+        GROUP_MIN_LEAVES leaves."""
         g = sph[chk["gate"]]
         # one extra test per obstacle pays for itself only over enough leaves
         if len(chk["leaves"]) < GROUP_MIN_LEAVES or any(sph[l]["frame"] != g["frame"] for l in chk["leaves"]):
             return None
-        R = max(float(np.linalg.norm(np.array(sph[l]["local"], dtype=np.float64) -
-                                     np.array(g["local"], dtype=np.float64))) + float(sph[l]["r"])
-                for l in chk["leaves"])
-        r = np.float32(R * (1.0 + 2.0 ** -16) + 1e-3)
-        return centre(chk["gate"]), float(np.nextafter(r, np.float32(np.inf)))
+        return centre(chk["gate"]), ball_of(chk["gate"], chk["leaves"])
 
     env = m["env_checks"]
     w("    uint64_t gate = 0;  /* bit k: env check k's gate sphere hit */")
@@ -388,7 +430,11 @@ def gen_robot_from(m: dict) -> str:
         if chk["direct"]:
             w("            if (g) ctx.hit();")
         else:
-            w("            if (g) {")
+            sides = split_pairs(chk)
+            ind = "            "
+            if sides is None:
+                w("            if (g) {")
+                ind += "    "
             used = []
             for a, b in chk["pairs"]:
                 for x in (a, b):
@@ -396,13 +442,32 @@ def gen_robot_from(m: dict) -> str:
                         used.append(x)
             for x in used:
                 c = centre(x)
-                w(f"                const float s{x}x = {c[0]}, s{x}y = {c[1]}, s{x}z = {c[2]};")
-            w("                bool h = false;")
-            for a, b in chk["pairs"]:
+                w(f"{ind}const float s{x}x = {c[0]}, s{x}y = {c[1]}, s{x}z = {c[2]};")
+            w(f"{ind}bool h = false;")
+
+            def pair(a, b, indent):
                 rs = flit(np.float32(sph[a]["r"]) + np.float32(sph[b]["r"]))
-                w(f"                h |= ctx.self(s{a}x, s{a}y, s{a}z, s{b}x, s{b}y, s{b}z, {rs});")
-            w("                if (h) ctx.hit();")
-            w("            }")
+                w(f"{indent}h |= ctx.self(s{a}x, s{a}y, s{a}z, s{b}x, s{b}y, s{b}z, {rs});")
+
+            if sides is None:
+                for a, b in chk["pairs"]:
+                    pair(a, b, ind)
+                w(f"{ind}if (h) ctx.hit();")
+                w("            }")
+            else:
+                # the spheres of one link one by one against the ball of the
+                # other link's: most are out of its reach on every lane
+                outer, inner, gate, R = sides
+                c = centre(gate)
+                w(f"{ind}const float cx = {c[0]}, cy = {c[1]}, cz = {c[2]};")
+                for x in outer:
+                    reach2 = np.nextafter(np.float32((R + float(sph[x]["r"])) ** 2), np.float32(np.inf))
+                    w(f"{ind}if (ctx.any(g && ctx.near_point(s{x}x, s{x}y, s{x}z, cx, cy, cz, {flit(reach2)}))) {{")
+                    for a, b in chk["pairs"]:
+                        if x in (a, b):
+                            pair(a, b, ind + "    ")
+                    w(f"{ind}}}")
+                w(f"{ind}if (g && h) ctx.hit();")
         w("            if (ctx.stop()) return;")
         w("        }")
         w("    }")

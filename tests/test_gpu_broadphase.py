@@ -124,3 +124,42 @@ def test_self_group_words(robot):
         reach = float(np.array(w >> 16, np.uint16).view(np.float16))
         rs = m["spheres"][a]["r"] + m["spheres"][b]["r"]
         assert rs + 0.99e-3 <= reach <= (rs + 1e-3) * 1.002
+
+
+@pytest.mark.parametrize("robot", ["panda", "fetch"])
+def test_split_groups_hold_every_pair(robot, oracle_robots):
+    """Self groups tested sphere by sphere against the other link's ball: every
+    pair of the group is emitted once, under its outer sphere, and on random
+    poses the ball's reach holds each inner sphere with most of the 1 mm pad
+    to spare (so a sphere out of reach collides with none of them)."""
+    import os
+    import re
+    from prrtc_amd.robots import limits, load_model
+    m = load_model(robot)
+    sph = m["spheres"]
+    here = os.path.join(os.path.dirname(__file__), "..", "prrtc_amd", "csrc", "robots")
+    text = open(os.path.join(here, robot + ".gen.h")).read()
+    by_label = {c["label"]: c for c in m["self_checks"]}
+    lo, span = limits(robot)
+    rng = np.random.default_rng(21)
+    c = np.asarray(oracle_robots[robot].fk((lo + span * rng.random((500, len(lo)), dtype=F32)).astype(F32)))
+    split = 0
+    for label, body in re.findall(r"/\* self: (.*?) \*/(.*?)(?=/\* self: |\Z)", text, re.S):
+        near = re.findall(r"near_point\(s(\d+)x, .*?, cx, cy, cz, ([0-9.e+-]+)f\)\)\) \{(.*?)\n            \}", body, re.S)
+        if not near:
+            continue
+        split += 1
+        chk = by_label[label]
+        pairs = []
+        for x, reach2, tests in near:
+            x = int(x)
+            got = [(int(a), int(b)) for a, b in re.findall(r"ctx\.self\(s(\d+)x, .*?, s(\d+)x, ", tests)]
+            assert all(x in p for p in got)
+            pairs += got
+            inner = [p[0] if p[1] == x else p[1] for p in got]
+            # the ball is about the gate of the inner spheres' side
+            gate = chk["gate"][1 if chk["pairs"][0][0] == x or x in [p[0] for p in chk["pairs"]] else 0]
+            hold = max(float(np.linalg.norm(c[:, y] - c[:, gate], axis=1).max()) + sph[y]["r"] for y in inner)
+            assert hold + sph[x]["r"] <= np.sqrt(float(reach2)) - 0.9e-3
+        assert sorted(pairs) == sorted(map(tuple, chk["pairs"]))
+    assert split >= 5
