@@ -64,3 +64,26 @@ def test_nearest_overflowing_distances(gpu):
         idx, d2 = run(gpu, trees, n, queries, w)
         assert np.array_equal(idx, np.zeros_like(idx)), (w, idx)
         assert np.all(np.isinf(d2)), (w, d2)
+
+
+@pytest.mark.parametrize("dof", [3, 7, 8, 14])
+@pytest.mark.parametrize("n,qpt", [(1, 2), (255, 3), (256, 4), (257, 5), (1024, 8), (1300, 13)])
+def test_tiles_equal_single_queries(dof, n, qpt, gpu):
+    """Queries that share a workgroup (many trees with several queries each)
+    get, bit for bit, what each gets alone: whole and short tiles, scans that
+    end inside a step, ties between lanes, steps and waves, and a query whose
+    distances are no numbers."""
+    rng = np.random.default_rng(dof * 100 + qpt)
+    cap = (n + 1023) // 1024 * 1024
+    n_trees = 530
+    trees = np.full((n_trees, dof, cap), np.nan, np.float32)
+    # few distinct coordinates: exact ties everywhere
+    trees[:, :, :n] = rng.integers(-2, 3, (n_trees, dof, n)).astype(np.float32) / 2
+    trees[::2, :, :n] += rng.normal(size=(len(trees[::2]), dof, n)).astype(np.float32)
+    queries = rng.uniform(-1.5, 1.5, (n_trees, qpt, dof)).astype(np.float32)
+    queries[3, 1, 0] = np.nan
+    alone = [run(gpu, trees, n, queries[:, j:j + 1], 4) for j in range(qpt)]
+    for w in (1, 3, 4):
+        idx, d2 = run(gpu, trees, n, queries, w)
+        for j, (i1, d1) in enumerate(alone):
+            assert np.array_equal(idx[:, j], i1[:, 0]) and np.array_equal(d2[:, j].view(np.int32), d1[:, 0].view(np.int32))
