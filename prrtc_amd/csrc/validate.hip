@@ -255,6 +255,107 @@ static bool all_finite(const float *p, size_t n) {
     return true;
 }
 
+// Copies n floats and says whether all are finite (one pass, without an
+// early exit, so that it vectorizes).
+static bool copy_finite(float *dst, const float *src, size_t n) {
+    uint32_t bad = 0;
+    for (size_t i = 0; i < n; i++) {
+        uint32_t b;
+        std::memcpy(&b, src + i, sizeof b);
+        std::memcpy(dst + i, &b, sizeof b);
+        bad |= (uint32_t)((b & 0x7f800000u) == 0x7f800000u);
+    }
+    return bad == 0;
+}
+
+// Device buffer, pinned staging and stream of a thread's host-buffer calls
+// (check_poses, validate_edges), kept between calls: three device
+// allocations and frees and three blocking copies were 110 of the 150 us of
+// a 4096-pose check.  At most kMost bytes of each, released when the thread
+// ends; a larger call brings its own (verdict_call).  Every call waits for
+// its own work, so a buffer is never in use when the thread's next call takes
+// it.
+struct HostCall {
+    static constexpr size_t kMost = 16u << 20;
+    char *dev = nullptr, *host = nullptr;
+    size_t bytes = 0;   // of each
+    hipStream_t stream = nullptr;
+    int device = -1;   // of the buffers and the stream
+
+    void release() {
+        if (dev) (void)hipFree(dev);
+        if (host) (void)hipHostFree(host);
+        if (stream) (void)hipStreamDestroy(stream);
+        dev = host = nullptr;
+        bytes = 0;
+        stream = nullptr;
+        device = -1;
+    }
+    ~HostCall() { release(); }
+    // Both buffers of at least n <= kMost bytes on the thread's current device.
+    void need(size_t n) {
+        int cur = 0;
+        PRRTC_HIP(hipGetDevice(&cur));
+        if (cur != device || n > bytes) {
+            release();
+            const size_t size = std::min(kMost, n + n / 2 + 65536);
+            PRRTC_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+            PRRTC_HIP(hipMalloc(&dev, size));
+            PRRTC_HIP(hipHostMalloc(&host, size, hipHostMallocDefault));
+            bytes = size;
+            device = cur;
+        }
+    }
+};
+
+static HostCall &host_call() {
+    static thread_local HostCall hc;
+    return hc;
+}
+
+// One verdict call on host buffers: packed scene and n_floats of input go up
+// in one copy, `launch` queues the kernel on the stream, n verdict bytes come
+// back.  Returns false, with nothing launched, if the input is not finite.
+template <class Launch>
+static bool verdict_call(const prrtc_scene *scene, const float *in, size_t n_floats, int n, uint8_t *out,
+                         Launch &&launch) {
+    const size_t scene_bytes = (sizeof(float) * scene_packed_floats(scene) + 255) & ~size_t(255);
+    const size_t in_bytes = (sizeof(float) * n_floats + 255) & ~size_t(255);
+    const size_t up = scene_bytes + in_bytes, total = up + (size_t)n;
+    if (total > HostCall::kMost) {
+        // the copies outweigh the allocations, and pinning as much would not pay
+        if (!all_finite(in, n_floats)) return false;
+        std::vector<float> packed(scene_packed_floats(scene));
+        scene_pack(scene, packed.data());
+        DevBuf<float> ds(packed.size()), di(n_floats);
+        DevBuf<uint8_t> dout(n);
+        PRRTC_HIP(hipMemcpy(ds.p, packed.data(), sizeof(float) * packed.size(), hipMemcpyHostToDevice));
+        PRRTC_HIP(hipMemcpy(di.p, in, sizeof(float) * n_floats, hipMemcpyHostToDevice));
+        launch(ds.p, di.p, dout.p, (hipStream_t)0);
+        PRRTC_HIP(hipMemcpy(out, dout.p, n, hipMemcpyDeviceToHost));
+        return true;
+    }
+    HostCall &hc = host_call();
+    hc.need(total);
+    if (!copy_finite(reinterpret_cast<float *>(hc.host + scene_bytes), in, n_floats)) return false;
+    struct Drain {   // a call that fails half way leaves nothing queued on the buffers
+        hipStream_t s;
+        bool done = false;
+        ~Drain() {
+            if (!done) (void)hipStreamSynchronize(s);
+        }
+    } drain{hc.stream};
+    scene_pack(scene, reinterpret_cast<float *>(hc.host));
+    PRRTC_HIP(hipMemcpyAsync(hc.dev, hc.host, scene_bytes + sizeof(float) * n_floats, hipMemcpyHostToDevice, hc.stream));
+    launch(reinterpret_cast<const float *>(hc.dev), reinterpret_cast<const float *>(hc.dev + scene_bytes),
+           reinterpret_cast<uint8_t *>(hc.dev + up), hc.stream);
+    PRRTC_HIP(hipMemcpyAsync(hc.host + up, hc.dev + up, (size_t)n, hipMemcpyDeviceToHost, hc.stream));
+    PRRTC_HIP(hipStreamSynchronize(hc.stream));
+    drain.done = true;
+    std::memcpy(out, hc.host + up, (size_t)n);
+    return true;
+}
+
 }  // namespace prrtc
 
 using namespace prrtc;
@@ -330,23 +431,21 @@ int prrtc_check_poses(int robot, const prrtc_scene *scene, const float *poses, i
             return PRRTC_EINVAL;
         }
         if (n == 0) return PRRTC_OK;
-        if (!all_finite(poses, (size_t)n * D)) {
+        const size_t f4 = (scene_packed_floats(scene) - 8) / 4;
+        const bool fits = scene_fits(f4);
+        const bool finite = fits ? verdict_call(scene, poses, (size_t)n * D, n, out_free,
+                                                [&](const float *ds, const float *dq, uint8_t *dout, hipStream_t st) {
+                                                    PRRTC_DISPATCH(robot, launch_check, ds, f4, dq, n, dout, st);
+                                                })
+                                 : all_finite(poses, (size_t)n * D);
+        if (!finite) {
             set_error("prrtc_check_poses: non-finite pose");
             return PRRTC_EINVAL;
         }
-        std::vector<float> packed(scene_packed_floats(scene));
-        scene_pack(scene, packed.data());
-        DevBuf<float> ds(packed.size()), dq((size_t)n * D);
-        DevBuf<uint8_t> dout(n);
-        PRRTC_HIP(hipMemcpy(ds.p, packed.data(), sizeof(float) * packed.size(), hipMemcpyHostToDevice));
-        PRRTC_HIP(hipMemcpy(dq.p, poses, sizeof(float) * n * D, hipMemcpyHostToDevice));
-        const size_t f4 = (packed.size() - 8) / 4;
-        if (!scene_fits(f4)) {
+        if (!fits) {
             set_error("prrtc_check_poses: scene tables exceed %zu bytes", kMaxLdsScene);
             return PRRTC_EINVAL;
         }
-        PRRTC_DISPATCH(robot, launch_check, ds.p, f4, dq.p, n, dout.p, (hipStream_t)0);
-        PRRTC_HIP(hipMemcpy(out_free, dout.p, n, hipMemcpyDeviceToHost));
         return PRRTC_OK;
     });
 }
@@ -360,23 +459,22 @@ int prrtc_validate_edges(int robot, const prrtc_scene *scene, const float *edges
             return PRRTC_EINVAL;
         }
         if (n == 0) return PRRTC_OK;
-        if (!all_finite(edges, (size_t)n * 2 * D)) {
+        const size_t f4 = (scene_packed_floats(scene) - 8) / 4;
+        const bool fits = scene_fits(f4);
+        const bool finite = fits ? verdict_call(scene, edges, (size_t)n * 2 * D, n, out_free,
+                                                [&](const float *ds, const float *de, uint8_t *dout, hipStream_t st) {
+                                                    PRRTC_DISPATCH(robot, launch_validate, ds, f4, de, n, granularity,
+                                                                   dout, st);
+                                                })
+                                 : all_finite(edges, (size_t)n * 2 * D);
+        if (!finite) {
             set_error("prrtc_validate_edges: non-finite edge endpoint");
             return PRRTC_EINVAL;
         }
-        std::vector<float> packed(scene_packed_floats(scene));
-        scene_pack(scene, packed.data());
-        DevBuf<float> ds(packed.size()), de((size_t)n * 2 * D);
-        DevBuf<uint8_t> dout(n);
-        PRRTC_HIP(hipMemcpy(ds.p, packed.data(), sizeof(float) * packed.size(), hipMemcpyHostToDevice));
-        PRRTC_HIP(hipMemcpy(de.p, edges, sizeof(float) * (size_t)n * 2 * D, hipMemcpyHostToDevice));
-        const size_t f4 = (packed.size() - 8) / 4;
-        if (!scene_fits(f4)) {
+        if (!fits) {
             set_error("prrtc_validate_edges: scene tables exceed %zu bytes", kMaxLdsScene);
             return PRRTC_EINVAL;
         }
-        PRRTC_DISPATCH(robot, launch_validate, ds.p, f4, de.p, n, granularity, dout.p, (hipStream_t)0);
-        PRRTC_HIP(hipMemcpy(out_free, dout.p, n, hipMemcpyDeviceToHost));
         return PRRTC_OK;
     });
 }
