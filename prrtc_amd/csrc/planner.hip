@@ -498,14 +498,25 @@ __device__ int plan_commit(const PlanDesc &d, PlanState *st, int p, PlanControl 
     int sz[2] = {st->size[0], st->size[1]};
     int status = kStatusRunning;
     int win_slot = -1, win_last = -1, win_t = 0, win_nn_o = 0;
+    // a slot's outcome (tree, flags, nearest, chain nodes; other tree's
+    // nearest); the next 64 slots' are read while these are committed
+    int4 next_m = make_int4(0, kSkip, 0, 0);
+    int next_o = 0;
+    auto read_outcome = [&](int s) {
+        next_m = make_int4(0, kSkip, 0, 0);
+        next_o = 0;
+        if (s < d.nnc) {
+            const int *m = d.meta + (size_t)s * 8;   // rows of 32 bytes
+            next_m = *reinterpret_cast<const int4 *>(m);
+            next_o = m[4];
+        }
+    };
+    read_outcome(lane);
     for (int c0 = 0; c0 < d.nnc && status == kStatusRunning && win_slot < 0; c0 += kWave) {
         const int s = c0 + lane;
         const bool valid = s < d.nnc;
-        int t = 0, flags = kSkip, nn = 0, n_ok = 0, nn_o = 0;
-        if (valid) {
-            const int *m = d.meta + (size_t)s * 8;
-            t = m[0]; flags = m[1]; nn = m[2]; n_ok = m[3]; nn_o = m[4];
-        }
+        const int t = next_m.x, flags = next_m.y, nn = next_m.z, n_ok = next_m.w, nn_o = next_o;
+        if (c0 + kWave < d.nnc) read_outcome(s + kWave);
         const bool skip = flags & kSkip;
         const bool ext_ok = flags & kExtOk;
         const bool conn = ext_ok && (flags & kConnected);
@@ -552,12 +563,26 @@ __device__ int plan_commit(const PlanDesc &d, PlanState *st, int p, PlanControl 
             float *tn = d.nodes + (size_t)t * D * d.cap;
             int *par = d.parent + (size_t)t * d.cap;
             float *rad = d.radii + (size_t)t * d.cap;
-            for (int i = 0; i < count; i++) {
-                const int idx = start + i;
+            // four nodes' rows in flight at a time (a lane's chain is up to
+            // max_ext + 1 nodes, each a trip to memory)
+            constexpr int kRows = D <= 8 ? 4 : 2;
+            for (int i0 = 0; i0 < count; i0 += kRows) {
+                float row[kRows][D];
 #pragma unroll
-                for (int k = 0; k < D; k++) tn[(size_t)k * d.cap + idx] = stage[(size_t)i * D + k];
-                par[idx] = i == 0 ? nn : idx - 1;
-                rad[idx] = FLT_MAX;
+                for (int j = 0; j < kRows; j++) {
+                    const int i = min(i0 + j, count - 1);
+#pragma unroll
+                    for (int k = 0; k < D; k++) row[j][k] = stage[(size_t)i * D + k];
+                }
+#pragma unroll
+                for (int j = 0; j < kRows; j++) {
+                    const int i = i0 + j, idx = start + i;
+                    if (i >= count) break;
+#pragma unroll
+                    for (int k = 0; k < D; k++) tn[(size_t)k * d.cap + idx] = row[j][k];
+                    par[idx] = i == 0 ? nn : idx - 1;
+                    rad[idx] = FLT_MAX;
+                }
             }
         }
         // sizes after this chunk
@@ -573,7 +598,9 @@ __device__ int plan_commit(const PlanDesc &d, PlanState *st, int p, PlanControl 
             const int wc = __builtin_amdgcn_readlane(count, first_conn);
             win_last = ws + wc - 1;
         }
-        __threadfence();   // this chunk's radii and nodes before the next chunk reads them
+        // this chunk's radii before the next chunk reads them, its nodes before
+        // the trace does: the same wave's, so no farther than L2
+        if (d.dd || win_slot >= 0) stores_done();
     }
     if (status == kStatusRunning && win_slot >= 0) {
         if (lane == 0) {
@@ -590,7 +617,7 @@ __device__ int plan_commit(const PlanDesc &d, PlanState *st, int p, PlanControl 
         st->status = status;
     }
     status = __builtin_amdgcn_readfirstlane(status);
-    __threadfence();
+    stores_done();   // every lane's; the store to next_slot below releases them
     if (lane == 0) {
         const unsigned long long key = ((unsigned long long)st->round << 32) | (unsigned)p;
         if (status == kStatusRunning) {
@@ -602,7 +629,8 @@ __device__ int plan_commit(const PlanDesc &d, PlanState *st, int p, PlanControl 
                 __hip_atomic_fetch_or(ctrl->aged_mask + (p >> 6), 1ull << (p & 63), __ATOMIC_RELAXED,
                                       __HIP_MEMORY_SCOPE_AGENT);
             store_release(&st->next_slot, 0);
-            __hip_atomic_fetch_or(ctrl->open_mask + (p >> 6), 1ull << (p & 63), __ATOMIC_RELEASE,
+            // only a hint where to claim: what a claim reads hangs on next_slot
+            __hip_atomic_fetch_or(ctrl->open_mask + (p >> 6), 1ull << (p & 63), __ATOMIC_RELAXED,
                                   __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_fetch_max(&ctrl->hot_key, key + (1ull << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
@@ -739,7 +767,7 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
                     open = live && __builtin_amdgcn_readfirstlane(__hip_atomic_load(
                                        &st->next_slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < nnc;
                 }
-                const int s = open ? wave_atomic_add(&st->next_slot, k) : nnc;
+                const int s = open ? wave_atomic_add<__ATOMIC_ACQUIRE>(&st->next_slot, k) : nnc;
                 if (s < 0 || s >= nnc) return -1;
                 got = min(k, nnc - s);
                 if (s + got == nnc && lane_id() == 0)
@@ -875,20 +903,23 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
                 meta[1] = kSkip;
                 meta[2] = meta[3] = meta[4] = 0;
             }
-            __threadfence();
+            stores_done();
         } else if (runs) {
             ctx.obs = scene_obs;
             ctx.wide_ok = !crowd && ctl[6] != 0;
             float *a = areas + (crowd ? (size_t)w * area : 0);
             run_task<Robot>(d, st, crowd ? s + w : s, ctx, a, lds_ext, crowd ? team_wave() : team_workgroup());
-            __threadfence();
+            stores_done();
         }
         // a shared task is written whole before its slot is counted
         if (!crowd) __syncthreads();
         // the wave that counts the round's last slot commits the round
         if (crowd ? runs : leader) {
-            const int prev = wave_atomic_add(&st->done_slots, 1);
-            if (prev == d.nnc - 1) run_commit<Robot>(d, st, p, ctrl, paths);
+            const int prev = wave_atomic_add<__ATOMIC_RELEASE>(&st->done_slots, 1);
+            if (prev == d.nnc - 1) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // the other slots' outcomes
+                run_commit<Robot>(d, st, p, ctrl, paths);
+            }
         }
         if (crowd) __syncthreads();   // ctl read by every wave before the leader claims again
     }

@@ -152,11 +152,33 @@ __device__ __forceinline__ void store_release(int *p, int v) {
     __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Lane-0 atomic, result broadcast to the wave.
+// Lane-0 atomic of the given order, result broadcast to the wave.
+template <int ORDER>
 __device__ __forceinline__ int wave_atomic_add(int *p, int v) {
     int r = 0;
-    if (lane_id() == 0) r = atomic_add_agent(p, v);
+    if (lane_id() == 0) r = __hip_atomic_fetch_add(p, v, ORDER, __HIP_MEMORY_SCOPE_AGENT);
     return __builtin_amdgcn_readfirstlane(r);
+}
+
+// Who waits for whom.  A release or acquire at agent scope writes back or
+// invalidates the XCD's L2 (about 4 us each with the chip at work), so each
+// hand-over has one of each and no fence beside them:
+//   * a task's stores are in L2 (stores_done) before its waves meet or, for a
+//     wave on its own, before it counts; the count of its slot releases them
+//     for the whole workgroup;
+//   * the wave that counts a round's last slot acquires (fence) and commits;
+//   * the commit's reset of next_slot releases the new round;
+//   * a claim acquires it.  The claim publishes nothing: what its workgroup
+//     wrote was released by the count of that task.
+// Before, a task ended with a fence and a count of both orders, a commit had
+// a fence per 64 slots, and a claim released too.  8 Fetch solves (256 slots)
+// 79.5 -> 64.5 ms, an uneven batch of 128 problems 156 -> 125 ms, one Panda
+// solve 195 -> 169 us.
+// Wait until this wave's stores have reached L2, and order them before what
+// the workgroup's other waves, or this wave's other lanes, do next.
+__device__ __forceinline__ void stores_done() {
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0), the other counters as they are
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
 }
 
 // ----------------------------------------------------------- planner math

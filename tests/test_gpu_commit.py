@@ -1,0 +1,35 @@
+"""Round commits at the sizes where one can go wrong -- slots around the
+64-slot blocks a commit reads ahead, chains around the rows it moves at a
+time, with the dynamic domain (a block reads radii the block before wrote) and
+without -- bit for bit against the oracle's round-synchronous planner on the
+point robot, whose arithmetic both share."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nnc", [1, 63, 64, 65, 130, 300])
+@pytest.mark.parametrize("dd", [0, 1])
+def test_commits_equal_the_oracle(nnc, dd, gpu, oracle_robots):
+    from oracle import oracle
+    from prrtc_amd import scenes as S
+    R = oracle_robots["sphere"]
+    # a wall with a gap far from the straight line: several rounds, chains of
+    # many lengths (range 0.3: up to 20 nodes and more)
+    sc = S.Scene.build(cuboids=[S.cuboid((0, -1.2, 0), (0, 0, 0), (0.2, 4.0, 6.0))],
+                       spheres=[S.sphere((2, 2, 1), 0.7)])
+    start, goal = np.array([-4, -1, 0.5], np.float32), np.array([4, -1.5, -0.5], np.float32)
+    oracle.set_fused(True)
+    try:
+        for rng_, rounds in ((0.3, 4), (2.5, 6), (0.3, 400)):
+            st = dict(num_new_configs=nnc, granularity=16, range=rng_, balance=2, tree_ratio=1.0, dynamic_domain=dd,
+                      dd_alpha=0.05, dd_radius=2.0, dd_min_radius=0.5, max_samples=20000, max_iters=rounds,
+                      seed=7)
+            res, path = gpu.solve("sphere", start, goal[None], sc, st)
+            _, want, opath = R.plan(sc, start, goal[None], st, mode=0)
+            got = (res["solved"], res["iters"], res["start_tree_size"], res["goal_tree_size"], res["edge_checks"])
+            assert got == (want.solved, want.iters, want.start_tree_size, want.goal_tree_size, want.edge_checks)
+            assert path.tobytes() == opath.tobytes()
+    finally:
+        oracle.set_fused(False)
