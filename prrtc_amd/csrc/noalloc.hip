@@ -116,7 +116,6 @@ int solve_noalloc(const HostProblem &hp, prrtc_result *out, float *path, int pat
     ctrl.path_cap = (int)std::min<size_t>(path_rows, INT32_MAX);
     ctrl.max_nnc = hp.st->num_new_configs;
     ctrl.prio_policy = kPrioOldest;
-    ctrl.wide_slots = plan_wide_slots();
     ctrl.crowd_above = 0;
     const unsigned long long masks[2] = {1ull, 1ull};   // problem 0 runs, round 1 open
     PRRTC_HIP(hipMemcpyAsync(dev + o_desc, &desc, sizeof desc, hipMemcpyHostToDevice, s));

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cfloat>
+#include <climits>
 #include <cstdlib>
 #include <map>
 #include <mutex>
@@ -73,7 +74,6 @@ struct TaskCtx : CheckCtx {
     // this wave's share of the obstacles (obs holds the whole staged scene)
     Share share;
     bool shared_stop; // the task runs on several waves: stop keys go through LDS
-    bool wide_ok;     // its chain passes may give each wave poses of its own
     __device__ __forceinline__ void share_gates(uint64_t &gate) {
         const int W = waves;
         if (W == 1) return;
@@ -173,7 +173,7 @@ __device__ __attribute__((always_inline)) void plan_task(const PlanDesc &d, Plan
         ctx.waves = gs;
         ctx.gbase = gw * gs;
     };
-    const bool wide_ok = __builtin_amdgcn_readfirstlane((int)ctx_in.wide_ok) != 0 && d.wide_from >= 0;
+    const int wide_from = __builtin_amdgcn_readfirstlane(d.wide_from >= 0 ? d.wide_from : INT_MAX);
     // pose groups for n poses: one pass where the waves allow it
     auto groups_for = [&](int n) {
         const int want = (n + kWave - 1) / kWave;
@@ -245,6 +245,7 @@ __device__ __attribute__((always_inline)) void plan_task(const PlanDesc &d, Plan
         // phase 1: the connect chain, pose j on sub-edge j / g at c_i + (j%g + 1) step
         const int G0 = __builtin_amdgcn_readfirstlane(d.wide_edge ? groups_for(g) : 1);
         const int passes = (g + kWave * G0 - 1) / (kWave * G0);
+        const int span = (g + G0 * passes - 1) / (G0 * passes);   // lanes of a wave that take a pose
         shape(G0);
         int phase = 0, p = 0, base = 0, total = 0, n_chain = 0, npass = 0, cpass = 0;
         unsigned n_ext = 0;
@@ -254,17 +255,18 @@ __device__ __attribute__((always_inline)) void plan_task(const PlanDesc &d, Plan
             int key = 0;
             bool dead;
             if (phase == 0) {
-                // virtual lane (lane, group) interleaved, so every pass of
-                // every group spans the whole edge
-                const int k = (lane * G0 + gw) * passes + p;
+                // each group takes a stretch of the edge of its own (a short
+                // one, so its positions fit small balls), interleaved over the
+                // passes
+                const int k = (gw * span + lane) * passes + p;
                 const float kk = (float)((k < g ? k : g - 1) + 1);
 #pragma unroll
                 for (int c = 0; c < D; c++) q[c] = fmaf(kk, delta[c], nnv[c]);
-                dead = k >= g;
+                dead = k >= g || lane >= span;
             } else {
                 // from chain pass wide_from on, the remaining poses spread
                 // over pose groups: group gw takes poses base + 64 gw + lane
-                shape(wide_ok && cpass >= d.wide_from ? groups_for(total - base) : 1);
+                shape(cpass >= wide_from ? groups_for(total - base) : 1);
                 const int j = base + gw * kWave + lane;
                 const int jj = j < total ? j : total - 1;
                 const int i = jj / g, k = jj % g;
@@ -742,7 +744,6 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
     while (true) {
         if (leader) {
             int p_out = -1, s_out = -1, n_out = 1, hot = 0, crowd = 0;   // p_out < 0: the workgroup leaves
-            int run_now = 0;   // running problems at the claim
             // Claim up to k consecutive slots of problem q if q runs and has
             // unclaimed slots in this round; returns the first slot (-1: none)
             // and their number in `got`.  A round the mask scan saw open is
@@ -788,7 +789,6 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
                 const int hp = __builtin_amdgcn_readfirstlane(hk ? (int)(hk & 0xffffffffu) : -1);
                 const int ph = hp >= 0 && hp < P ? hp : -1;
                 const MaskScan ms = scan_masks(ctrl, words, cursor, ph);
-                run_now = ms.running;
                 // the running problems can use at most running * nnc
                 // workgroups: the rest leave, so a few long problems do not
                 // share their counters with the whole grid
@@ -868,7 +868,6 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
                 ctl[3] = prio;
                 ctl[4] = crowd;
                 ctl[5] = halt;
-                ctl[6] = (long long)run_now * max_nnc <= ctrl->wide_slots;
             }
         }
         __syncthreads();
@@ -906,7 +905,6 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
             stores_done();
         } else if (runs) {
             ctx.obs = scene_obs;
-            ctx.wide_ok = !crowd && ctl[6] != 0;
             float *a = areas + (crowd ? (size_t)w * area : 0);
             run_task<Robot>(d, st, crowd ? s + w : s, ctx, a, lds_ext, crowd ? team_wave() : team_workgroup());
             stores_done();
@@ -991,7 +989,6 @@ void k_round_tasks(const PlanDesc *__restrict__ descs, PlanState *states, int ma
     ctx.independent = false;
     ctx.gbuf = gbuf;
     bind_scene(d.scene, d.scene_f4, lds, ctx.obs);
-    ctx.wide_ok = false;   // a grid of every running problem's slots: throughput-bound
     plan_task<Robot>(d, st, s, ctx, a, a + (lds_ext + 1) * D, a + (lds_ext + 5) * D,
                      reinterpret_cast<int *>(a + (lds_ext + 5) * D + 2 * kMaxTaskWaves), team_workgroup());
 }
@@ -1138,32 +1135,23 @@ void block_upload_image(const HostProblem &hp, const BlockLayout &L, char *host)
     std::memcpy(ini + D, hp.goals, sizeof(float) * (size_t)hp.n_goals * D);
 }
 
-// Chain pass from which a task's waves may take distinct poses (negative:
-// never; PRRTC_WIDE_FROM overrides the robot's default).  Whether they do is
-// decided per task (PlanControl::wide_slots).  A wide pass saves the
-// forward kinematics the waves of a shared pass compute alike and the gate
-// exchange; Fetch's checks are dominated by its bounded leaf groups rather
-// than its kinematics, and its solves measured slower with wide passes (48
-// C2 problems alone at nnc 128: 748 -> 923 ms of kernel; the mix's Fetch
-// problems 197 -> 214 ms), Panda's and Baxter's faster (C0 16.5 -> 14.6 ms,
-// the C1 plans 1582 -> 1461 ms, the mix's Panda 2236 -> 2110 and Baxter
-// 1016 -> 965 ms).
-static int wide_from(int robot) {
+// Chain pass from which a task's waves take distinct poses (PRRTC_WIDE_FROM;
+// negative: never).  Such a pass computes no pose's kinematics and balls
+// twice and needs no gate exchange, and each wave's stretch of the chain is
+// short, so its lists of near obstacles and groups are too; sharing 64 poses
+// splits only the tests on the lists, which are the smaller part.  From the
+// first pass, for every robot and however many problems run: 8 Fetch solves
+// 106 -> 99 ms (14 -> 12, 142 -> 136 on other problems), a batch of 128 mixed
+// problems 122 -> 98 ms (147 -> 124, 134 -> 101) against wide passes for
+// Panda and Baxter while half the CUs are free; never: a Panda solve 121 ->
+// 165 us.
+static int wide_from() {
     static const int env = [] {
         const char *e = std::getenv("PRRTC_WIDE_FROM");
-        return e ? std::atoi(e) : INT32_MIN;
+        return e ? std::atoi(e) : 0;
     }();
-    if (env != INT32_MIN) return env;
-    return robot == PRRTC_ROBOT_FETCH ? -1 : 0;
+    return env;
 }
-
-// Chain passes go wide only while the running problems' rounds leave half
-// the CUs free: such rounds wait for their slowest task.  A round that fills
-// the machine is bound by throughput, and the poses a wide pass adds (past a
-// chain's first collision, on waves without poses) cost more than its
-// shorter passes save (the 256-slot C2 plain solves 15% slower, the C2
-// batch's tail 13%).
-int plan_wide_slots() { return num_cus() / 2; }
 
 // Whether a steered edge of more than 64 poses spreads them over pose groups
 // (PRRTC_WIDE_EDGE overrides).
@@ -1177,7 +1165,7 @@ static int wide_edge() {
 
 void fill_desc(PlanDesc &d, const HostProblem &hp, const BlockLayout &L, char *dev) {
     d = PlanDesc{};
-    d.wide_from = wide_from(hp.robot);
+    d.wide_from = wide_from();
     d.wide_edge = wide_edge();
     d.nnc = hp.st->num_new_configs;
     d.g = hp.st->granularity;
@@ -1461,7 +1449,6 @@ static void start_group(GroupRun &gr, int path_cap) {
     hc->path_stride = D;
     for (int i = 0; i < P; i++) hc->max_nnc = std::max(hc->max_nnc, probs[i].st->num_new_configs);
     hc->prio_policy = kPrioOldest;
-    hc->wide_slots = plan_wide_slots();
     hc->crowd_above = P > 1 ? largest([&](int r) { return plan_crowd_above(r, hc->max_nnc); }) : 0;
     // --- upload (descs, masks and control in one copy; scenes and init rows
     // per problem): the control block is complete before the copy is queued

@@ -46,8 +46,6 @@ BlockLayout block_layout(const HostProblem &hp);
 void block_upload_image(const HostProblem &hp, const BlockLayout &L, char *host);
 // Fills a PlanDesc whose buffers live in the device block at `dev`.
 void fill_desc(PlanDesc &d, const HostProblem &hp, const BlockLayout &L, char *dev);
-// PlanControl::wide_slots of a launch on this device
-int plan_wide_slots();
 
 // Launch shapes of a robot's persistent planner grids: the value set by
 // prrtc_set_tuning, else an environment variable, else the default.
