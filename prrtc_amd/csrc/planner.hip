@@ -197,27 +197,24 @@ __device__ __attribute__((always_inline)) void plan_task(const PlanDesc &d, Plan
     int *stopw = task_stop_words();
     if (tid == 0 && tm.waves > 1) stopw[0] = stopw[1] = 0x7fffffff;   // read only after the next barrier
 
-    // tree choice and Halton sample (uniform across the workgroup)
+    // tree choice and Halton sample (the same on every wave)
     const int t = choose_tree(d, s, iter, d.tprev[s], n0, n1);
     const int o = 1 - t;
     float *hs = d.halton + (size_t)s * 3 * D;
-    float sample[D], h_n[D], h_d[D];
+    // one dimension per lane (lanes past D repeat the last): D dimensions'
+    // loads and divisions at once instead of one after another
+    const int hk = lane < D ? lane : D - 1;
+    float h_b = hs[hk], h_n = hs[D + hk], h_d = hs[2 * D + hk];
+    const float u = halton_step(h_b, h_n, h_d);
+    float sample[D];
 #pragma unroll
-    for (int k = 0; k < D; k++) {
-        float b = hs[k], n = hs[D + k], dd = hs[2 * D + k];
-        const float u = halton_step(b, n, dd);
-        h_n[k] = n;
-        h_d[k] = dd;
-        sample[k] = fmaf(u, Robot::span(k), Robot::lower(k));     // Robots.hh scale_cfg
-    }
-    // every wave has read the slot's Halton state and tree before thread 0
-    // advances them
+    for (int k = 0; k < D; k++)
+        sample[k] = fmaf(lane_value(u, k), Robot::span(k), Robot::lower(k));     // Robots.hh scale_cfg
+    // every wave has read the slot's Halton state and tree before the first
+    // one advances them
     if (tm.waves > 1) tm.sync();
-    if (tid == 0) {
-#pragma unroll
-        for (int k = 0; k < D; k++) { hs[D + k] = h_n[k]; hs[2 * D + k] = h_d[k]; }
-        d.tprev[s] = t;
-    }
+    if (tid < D) { hs[D + tid] = h_n; hs[2 * D + tid] = h_d; }
+    if (tid == 0) d.tprev[s] = t;
 
     // nearest node in the target tree (pRRTC.cu:384-418)
     const float *tn = d.nodes + (size_t)t * D * d.cap;

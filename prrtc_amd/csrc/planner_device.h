@@ -204,7 +204,7 @@ __device__ __forceinline__ int choose_tree(const PlanDesc &d, int slot, int iter
     return t;
 }
 
-// Incremental Halton step of one dimension (pRRTC.cu:81-105); uniform.
+// Incremental Halton step of one dimension (pRRTC.cu:81-105).
 __device__ __forceinline__ float halton_step(float &b, float &n, float &dd) {
 #pragma clang fp contract(off)
     const float xf = dd - n;
