@@ -216,7 +216,11 @@ static void launch_scene_kernel(void (*k)(KArgs...), dim3 grid, size_t scene_f4,
 template <class Robot>
 static void launch_validate(const float *d_scene, size_t scene_f4, const float *d_edges, int n, int g,
                             uint8_t *d_out, hipStream_t st) {
-    const int grid = std::max(1, std::min(n, num_cus() * 16));
+    // three workgroups for each of the eight waves a CU holds: edges take
+    // uneven time, and the last ones even out; each workgroup stages the
+    // scene, so many more would cost.  Against two: 10k Fetch edges 82 -> 79
+    // us (139 -> 131 on another scene), 30k Baxter edges 260 -> 249 us.
+    const int grid = std::max(1, std::min(n, num_cus() * 24));
     launch_scene_kernel(k_validate_edges<Robot>, dim3(grid), scene_f4, st, d_scene, (int)scene_f4, d_edges,
                         n, g, d_out);
 }
