@@ -924,21 +924,21 @@ void k_plan(const PlanDesc *__restrict__ descs, PlanState *states, PlanControl *
 template <class Robot>
 __device__ __forceinline__ void init_problem(const PlanDesc &d, PlanState *st) {
     constexpr int D = Robot::DOF;
-    const int lane = lane_id();
-    for (int i = lane; i < 1 + d.n_goals; i += kWave) {
+    const int tid = threadIdx.x, nt = blockDim.x;
+    for (int i = tid; i < 1 + d.n_goals; i += nt) {
         const int t = i == 0 ? 0 : 1, idx = i == 0 ? 0 : i - 1;
         for (int k = 0; k < D; k++) d.nodes[(size_t)t * D * d.cap + (size_t)k * d.cap + idx] = d.init[(size_t)i * D + k];
         d.parent[(size_t)t * d.cap + idx] = idx;
         d.radii[(size_t)t * d.cap + idx] = FLT_MAX;
     }
-    for (int s = lane; s < d.nnc; s += kWave) {
+    for (int s = tid; s < d.nnc; s += nt) {
         float b[16];
         halton_bases(d.seed, s, D, b);
         float *hs = d.halton + (size_t)s * 3 * D;
         for (int k = 0; k < D; k++) { hs[k] = b[k]; hs[D + k] = 0.0f; hs[2 * D + k] = 1.0f; }
         d.tprev[s] = 0;
     }
-    if (lane == 0) {
+    if (tid == 0) {
         *st = PlanState{};
         st->status = kStatusRunning;
         st->round = 1;
@@ -948,8 +948,13 @@ __device__ __forceinline__ void init_problem(const PlanDesc &d, PlanState *st) {
     }
 }
 
+// Threads of a problem's setup: a slot's shuffle is some 2 us of dependent
+// arithmetic, so the slots are spread over a whole workgroup (256 slots of
+// Fetch on one wave 11.0 us, on four 6.2 us; 128 of Panda 7.6 and 6.5 us).
+constexpr int kInitThreads = 256;
+
 template <class Robot>
-__global__ __launch_bounds__(kWave) void k_plan_init(const PlanDesc *__restrict__ descs, PlanState *states,
+__global__ __launch_bounds__(kInitThreads) void k_plan_init(const PlanDesc *__restrict__ descs, PlanState *states,
                                                      const int *__restrict__ list) {
     const int e = list ? list[blockIdx.x] : (int)blockIdx.x;   // problem (table entry) to set up
     const PlanDesc &d = descs[e];
@@ -1216,7 +1221,7 @@ void launch_plan_init(int robot, const PlanDesc *d_desc, PlanState *d_state, con
     if (n <= 0) return;
     switch (robot) {
 #define PRRTC_INIT_CASE(ID, R) \
-    case ID: hipLaunchKernelGGL(k_plan_init<R>, dim3(n), dim3(kWave), 0, s, d_desc, d_state, d_list); break;
+    case ID: hipLaunchKernelGGL(k_plan_init<R>, dim3(n), dim3(kInitThreads), 0, s, d_desc, d_state, d_list); break;
         PRRTC_FOR_EACH_ROBOT(PRRTC_INIT_CASE)
         PRRTC_INIT_CASE(kRobotMixed, AnyRobot)
 #undef PRRTC_INIT_CASE
