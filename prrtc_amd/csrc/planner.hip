@@ -40,7 +40,7 @@ __device__ __forceinline__ int across_waves(int v, bool want_min, int *buf, int 
 
 // Check context of a planner task.  The task's waves validate the same 64
 // poses per pass and split the obstacle tables between them (each wave's
-// `obs` is one slice), so a pass costs a fraction of one wave's work; a
+// `share`), so a pass costs a fraction of one wave's work; a
 // pose's gate bits are ORed across the waves before the leaf checks, and
 // the waves' collision flags are combined after the pass.  A gate hits iff
 // some obstacle hits it, whichever wave tests that obstacle, so the verdicts
@@ -57,7 +57,7 @@ __device__ __forceinline__ int across_waves(int v, bool want_min, int *buf, int 
 //
 // Self-collision groups, which need no obstacles, are dealt out instead:
 // group j goes to wave j mod W (`mine`), and a hit on any wave ends the pass
-// on all of them through the same word.  Every group is still tested by one
+// on all of them through the same word.  Every group in reach is tested by one
 // wave for every live lane, so the verdicts are unchanged.
 // The two words live in static LDS, so every access is a plain LDS
 // instruction; only a task of the whole workgroup uses them.
