@@ -42,3 +42,31 @@ def test_chain_passes_shared_or_apart(gpu):
     base = T.solve_digests()
     assert T._child({"PRRTC_WIDE_FROM": "-1"}) == base
     assert T._child({"PRRTC_WIDE_FROM": "2"}) == base
+
+
+@pytest.mark.parametrize("robot", ["fetch", "baxter"])
+def test_largest_scene_and_chains(robot, gpu):
+    """The most LDS a planner workgroup can ask for: full obstacle tables (64
+    KiB, and half as much for their balls) and chains of nearly 255 steps,
+    alone and in a batch of two robots (one grid laid out for the largest)."""
+    from prrtc_amd import scenes as S
+    from prrtc_amd.robots import limits
+    rng = np.random.default_rng(2)
+    sc = S.Scene.build(z_cuboids=[S.cuboid(rng.uniform(3, 5, 3), (0, 0, 1.0), (0.05, 0.05, 0.05)) for _ in range(1024)])
+    lo, span = limits(robot)
+    q = (lo + span * rng.random((4096, len(lo)), dtype=np.float32)).astype(np.float32)
+    q = q[gpu.check_poses(robot, sc, q)][:2]
+    st = dict(num_new_configs=16, granularity=8, range=float(np.linalg.norm(span)) / 250, balance=2, tree_ratio=1.0,
+              dynamic_domain=0, max_samples=20000, max_iters=3, seed=1)
+    p = {"robot": robot, "start": q[0], "goals": q[1][None], "scene": sc}
+    other = "fetch" if robot == "baxter" else "baxter"
+    lo2, span2 = limits(other)
+    q2 = (lo2 + span2 * rng.random((4096, len(lo2)), dtype=np.float32)).astype(np.float32)
+    q2 = q2[gpu.check_poses(other, sc, q2)][:2]
+    p2 = {"robot": other, "start": q2[0], "goals": q2[1][None], "scene": sc}
+    alone, path = gpu.solve(robot, p["start"], p["goals"], sc, st)
+    res, paths, _ = gpu.solve_batch([p, p2], [st, dict(st, range=float(np.linalg.norm(span2)) / 250)])
+    for k in ("solved", "status", "iters", "start_tree_size", "goal_tree_size", "edge_checks", "path_nodes"):
+        assert alone[k] == res[0][k]
+    assert path.tobytes() == paths[0].tobytes()
+    assert alone["start_tree_size"] + alone["goal_tree_size"] > 2
