@@ -381,14 +381,75 @@ __device__ __forceinline__ void env_hits(const Obstacles &o, Share sh, const flo
     for (int n = 0; n < N; n++) hit[n] = m[n] < 0.0f;
 }
 
+// The same for poses that have nothing to do with each other (SpreadCtx):
+// their balls would rule out little, so every obstacle is tested in turn, a
+// capsule or cuboid unless it is out of a sphere's reach on every live lane.
+template <int N, bool LOCAL>
+__device__ __forceinline__ void env_hits_each(const Obstacles &o, const float (&x)[N], const float (&y)[N],
+                                              const float (&z)[N], const float (&r)[N], bool on, bool (&hit)[N]) {
+#pragma clang fp contract(off)
+    float m[N];
+#pragma unroll
+    for (int n = 0; n < N; n++) m[n] = __builtin_huge_valf();
+    auto far = [&](const float4 &b, int n) {   // on every active lane
+        const float rb = r[n] + b.w;
+        return ballot(!(sq3(x[n] - b.x, y[n] - b.y, z[n] - b.z) > rb * rb)) == 0;
+    };
+    if (on) {
+        for (int i = 0; i < o.n_sph; i++) {
+            const float4 s = ld_obs<LOCAL>(o.sph + i);
+#pragma unroll
+            for (int n = 0; n < N; n++) m[n] = fminf(m[n], sphere_test(s, x[n], y[n], z[n], r[n]));
+        }
+        for (int i = 0; i < o.n_cap; i++) {
+            const float4 p = ld_obs<LOCAL>(o.cap + 2 * i), v = ld_obs<LOCAL>(o.cap + 2 * i + 1),
+                         b = ld_obs<LOCAL>(o.ball + i);
+#pragma unroll
+            for (int n = 0; n < N; n++) {
+                if (far(b, n)) continue;
+                m[n] = fminf(m[n], capsule_test(p, v, x[n], y[n], z[n], r[n]));
+            }
+        }
+        for (int i = 0; i < o.n_zcap; i++) {
+            const float4 p = ld_obs<LOCAL>(o.zcap + 2 * i), v = ld_obs<LOCAL>(o.zcap + 2 * i + 1);
+#pragma unroll
+            for (int n = 0; n < N; n++) m[n] = fminf(m[n], z_capsule_test(p, v, x[n], y[n], z[n], r[n]));
+        }
+        for (int i = 0; i < o.n_cub; i++) {
+            const float4 p = ld_obs<LOCAL>(o.cub + 4 * i), a1 = ld_obs<LOCAL>(o.cub + 4 * i + 1),
+                         a2 = ld_obs<LOCAL>(o.cub + 4 * i + 2), a3 = ld_obs<LOCAL>(o.cub + 4 * i + 3);
+            const float4 b = make_float4(p.x, p.y, p.z, a3.w);
+#pragma unroll
+            for (int n = 0; n < N; n++) {
+                if (far(b, n)) continue;
+                m[n] = fminf(m[n], cuboid_test(p, a1, a2, a3, x[n], y[n], z[n], r[n]));
+            }
+        }
+        for (int i = 0; i < o.n_zcub; i++) {
+            const float4 p = ld_obs<LOCAL>(o.zcub + 4 * i), a1 = ld_obs<LOCAL>(o.zcub + 4 * i + 1),
+                         a2 = ld_obs<LOCAL>(o.zcub + 4 * i + 2);
+            const float4 b = make_float4(p.x, p.y, p.z, ld_obs<LOCAL>(o.zcub + 4 * i + 3).w);
+#pragma unroll
+            for (int n = 0; n < N; n++) {
+                if (far(b, n)) continue;
+                m[n] = fminf(m[n], z_cuboid_test(p, a1, a2, x[n], y[n], z[n], r[n]));
+            }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < N; n++) hit[n] = m[n] < 0.0f;
+}
+
 // Whether any of N spheres (the leaves of one link) hits an obstacle, on each
 // live lane.  The spheres of every lane lie in one ball about `c`, `reach`
 // its radius.  One running minimum serves the group (some value < 0 iff their
 // minimum is).  EARLY: the wave leaves once every live lane has a hit.
-template <int N, bool EARLY, bool LOCAL>
+// skip(ball) says (wave-uniformly) that an obstacle on the list is out of the
+// whole group's reach all the same.
+template <int N, bool EARLY, bool LOCAL, class Skip>
 __device__ __forceinline__ bool env_group(const Obstacles &o, Share sh, const float (&x)[N], const float (&y)[N],
                                           const float (&z)[N], const float (&r)[N], bool on, const WaveBall &c,
-                                          float reach) {
+                                          float reach, Skip skip) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & (kWave - 1);
     const int mine = (o.count() - sh.part + (1 << sh.shift) - 1) >> sh.shift;
@@ -402,6 +463,7 @@ __device__ __forceinline__ bool env_group(const Obstacles &o, Share sh, const fl
             // of a link's spheres near an obstacle most are out of its reach
             // on every lane; the exact test costs three times this one
             const float4 ob = obstacle_ball<LOCAL>(o, i);
+            if (skip(ob)) continue;
             test_obstacle<N, LOCAL, true, false>(o, i, x, y, z, r, m, [&](int n) {
                 const float rb = r[n] + ob.w;
                 return ballot(!(sq3(x[n] - ob.x, y[n] - ob.y, z[n] - ob.z) > rb * rb)) == 0;
@@ -429,19 +491,22 @@ __device__ __forceinline__ bool env_leaves(const Obstacles &o, Share sh, const f
         rmax = fmaxf(rmax, r[n]);
     }
     c.r = ball_radius(__int_as_float((int)d), on);
-    return env_group<N, EARLY, LOCAL>(o, sh, x, y, z, r, on, c, c.r + rmax);
+    return env_group<N, EARLY, LOCAL>(o, sh, x, y, z, r, on, c, c.r + rmax, [](const float4 &) { return false; });
 }
 
 // env_group for spheres that lie in the ball (gx, gy, gz; gr) on every lane
 // -- the leaves of one link, bounded about the link's gate centre with a
-// 1 mm pad by the generator.
-template <int N, bool EARLY, bool LOCAL>
+// 1 mm pad by the generator.  SPREAD: the lanes' balls lie far apart, so the
+// ball around them lists most obstacles; each is asked of the lanes' own first.
+template <int N, bool EARLY, bool LOCAL, bool SPREAD = false>
 __device__ __forceinline__ bool env_leaves_bounded(const Obstacles &o, Share sh, const float (&x)[N],
                                                    const float (&y)[N], const float (&z)[N], const float (&r)[N],
                                                    bool on, float gx, float gy, float gz, float gr) {
 #pragma clang fp contract(off)
     const WaveBall c = wave_ball(gx, gy, gz, on, ballot(on));
-    return env_group<N, EARLY, LOCAL>(o, sh, x, y, z, r, on, c, c.r + gr);
+    return env_group<N, EARLY, LOCAL>(o, sh, x, y, z, r, on, c, c.r + gr, [&](const float4 &b) {
+        return SPREAD && ballot(on && in_reach(b, WaveBall{gx, gy, gz, 0.0f}, gr)) == 0;
+    });
 }
 
 // sphere_sphere_self_collision (utils.cuh:83-86) with the radius sum folded.
@@ -585,12 +650,33 @@ struct CheckCtx {
     }
 };
 
+// Check context of a pass of poses that have nothing to do with each other:
+// no balls over the wave, neither for the gates nor for the self-collision
+// groups.
+struct SpreadCtx : CheckCtx {
+    template <int N>
+    __device__ __forceinline__ void env_gates(int, const float (&x)[N], const float (&y)[N], const float (&z)[N],
+                                              const float (&r)[N], bool (&hit)[N]) const {
+        env_hits_each<N, false>(obs, x, y, z, r, live(), hit);
+    }
+    __device__ __forceinline__ void fixed_gate(int, float, float, float) {}
+    template <int NS>
+    __device__ __forceinline__ void self_near(const uint32_t *) { self_groups_own<NS>(Share{}, near); }
+    template <int N, bool EARLY>
+    __device__ __forceinline__ bool env_any_bounded(const float (&x)[N], const float (&y)[N], const float (&z)[N],
+                                                    const float (&r)[N], bool on, float gx, float gy, float gz,
+                                                    float gr) const {
+        return env_leaves_bounded<N, EARLY, false, true>(obs, Share{}, x, y, z, r, on, gx, gy, gz, gr);
+    }
+};
+
 // ---------------------------------------------------------------------------
 // robots
 
 struct SphereRobot {     // Robots.hh:190-237; fkcc<Sphere>, utils.cuh:330-334
     static constexpr int DOF = 3;
     static constexpr int NSPHERES = 1;
+    static constexpr float kSpread = 2.0f;   // in its cube of side 10
     __host__ __device__ static constexpr float lower(int) { return -5.0f; }
     __host__ __device__ static constexpr float span(int) { return 10.0f; }
     template <class Ctx>
@@ -608,8 +694,10 @@ struct SphereRobot {     // Robots.hh:190-237; fkcc<Sphere>, utils.cuh:330-334
     }
 };
 
-#define PRRTC_GEN_ROBOT(NAME, NS)                                                              \
+// kSpread (see launch_check): joint distance at which poses count as unrelated
+#define PRRTC_GEN_ROBOT(NAME, NS, SPREAD)                                                      \
     struct NAME##Robot {                                                                       \
+        static constexpr float kSpread = SPREAD;                                               \
         static constexpr int DOF = gen::NS::DOF;                                               \
         static constexpr int NSPHERES = gen::NS::NSPHERES;                                     \
         __host__ __device__ static constexpr float lower(int i) { return gen::NS::lower(i); } \
@@ -622,10 +710,10 @@ struct SphereRobot {     // Robots.hh:190-237; fkcc<Sphere>, utils.cuh:330-334
             gen::NS::fk_spheres(q, out);                                                       \
         }                                                                                      \
     };
-PRRTC_GEN_ROBOT(Panda, panda)
-PRRTC_GEN_ROBOT(Fetch, fetch)
-PRRTC_GEN_ROBOT(Baxter, baxter)
-PRRTC_GEN_ROBOT(Ur5, ur5)
+PRRTC_GEN_ROBOT(Panda, panda, 2.2f)
+PRRTC_GEN_ROBOT(Fetch, fetch, 1.6f)
+PRRTC_GEN_ROBOT(Baxter, baxter, 4.2f)
+PRRTC_GEN_ROBOT(Ur5, ur5, 3.5f)
 #undef PRRTC_GEN_ROBOT
 
 // Every robot the library is built for, as X(id, struct): the one list the

@@ -32,12 +32,15 @@ __global__ __launch_bounds__(kWave) void k_fk_spheres(const float *__restrict__ 
     Robot::fk_spheres(q, out + (size_t)i * Robot::NSPHERES * 3);
 }
 
-template <class Robot>
+// Lane l of a wave takes pose base + l.  Ctx: CheckCtx where the poses of a
+// wave lie together (a path's), SpreadCtx where they have nothing to do with
+// each other (samples); the verdicts are the same (see launch_check).
+template <class Robot, class Ctx>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void k_check_poses(const float *__restrict__ scene, int scene_f4,
                                                        const float *__restrict__ poses, int n,
                                                        uint8_t *__restrict__ out) {
     extern __shared__ float4 lds_scene[];
-    CheckCtx ctx;
+    Ctx ctx;
     ctx.independent = true;
     ctx.key = 0;
     bind_scene(scene, scene_f4, lds_scene, ctx.obs);
@@ -225,13 +228,46 @@ static void launch_validate(const float *d_scene, size_t scene_f4, const float *
                         n, g, d_out);
 }
 
+// Whether the poses (on the host) are samples rather than paths: most blocks of
+// 64, at most 64 of them asked, hold a pose farther than `apart` (2-norm over
+// the joints) from their first, among three of them.
+static bool poses_apart(const float *poses, int n, int dof, float apart) {
+    const int blocks = (n + kWave - 1) / kWave, asked = std::min(blocks, 64);
+    int far = 0;
+    for (int j = 0; j < asked; j++) {
+        const size_t first = (size_t)((long long)blocks * j / asked) * kWave;
+        const size_t last = std::min(first + kWave, (size_t)n) - 1;
+        float most = 0.0f;
+        for (int k = 1; k <= 3; k++) {
+            const float *p = poses + first * dof, *q = poses + (first + (last - first) * k / 3) * dof;
+            float d2 = 0.0f;
+            for (int d = 0; d < dof; d++) d2 += (q[d] - p[d]) * (q[d] - p[d]);
+            most = std::max(most, d2);
+        }
+        far += most > apart * apart;
+    }
+    return 2 * far > asked;
+}
+
+// Poses of a path are checked like an edge's, by balls over the wave; samples
+// pose by pose (SpreadCtx), since balls around them rule out little and cost
+// their own forming and a branch per gate and obstacle.  kSpread is the length
+// of a 64-pose path at which both take the same time: Panda 2 to 2.5, Fetch
+// 1.5 to 2, Baxter 4 to 5, UR5 3 to 5, over scenes of 12 to 4096 obstacles.
+// 4096 uniform poses by balls and pose by pose: Panda, 72 obstacles 207 and 157
+// us, 1000 spheres 1182 and 860; Baxter, 32 boxes 73 and 50 us, 1000 spheres
+// 1084 and 648.  64 paths of 0.5 rad: Panda, 72 obstacles 26 and 48 us, 1000
+// spheres 73 and 236.
 template <class Robot>
-static void launch_check(const float *d_scene, size_t scene_f4, const float *d_poses, int n, uint8_t *d_out,
+static void launch_check(const float *d_scene, size_t scene_f4, const float *d_poses, int n, bool apart, uint8_t *d_out,
                          hipStream_t st) {
     const int blocks = std::max(1, std::min((n + kWave - 1) / kWave, num_cus() * 16));
-    launch_scene_kernel(k_check_poses<Robot>, dim3(blocks), scene_f4, st, d_scene, (int)scene_f4, d_poses,
-                        n, d_out);
+    launch_scene_kernel(apart ? k_check_poses<Robot, SpreadCtx> : k_check_poses<Robot, CheckCtx>, dim3(blocks), scene_f4,
+                        st, d_scene, (int)scene_f4, d_poses, n, d_out);
 }
+
+template <class Robot>
+static void spread_of(float &out) { out = Robot::kSpread; }
 
 // Scenes are staged whole into LDS: at most kMaxLdsScene bytes of tables
 // (4096 float4: e.g. 1024 cuboids or 4096 spheres).
@@ -439,7 +475,10 @@ int prrtc_check_poses(int robot, const prrtc_scene *scene, const float *poses, i
         const bool fits = scene_fits(f4);
         const bool finite = fits ? verdict_call(scene, poses, (size_t)n * D, n, out_free,
                                                 [&](const float *ds, const float *dq, uint8_t *dout, hipStream_t st) {
-                                                    PRRTC_DISPATCH(robot, launch_check, ds, f4, dq, n, dout, st);
+                                                    float spread = 0.0f;
+                                                    PRRTC_DISPATCH(robot, spread_of, spread);
+                                                    const bool apart = poses_apart(poses, n, D, spread);
+                                                    PRRTC_DISPATCH(robot, launch_check, ds, f4, dq, n, apart, dout, st);
                                                 })
                                  : all_finite(poses, (size_t)n * D);
         if (!finite) {

@@ -54,6 +54,29 @@ def test_edges_against_oracle(robot, counts, gpu, oracle_robots):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("robot", ["panda", "fetch", "baxter", "ur5"])
+@pytest.mark.parametrize("counts", COUNTS, ids=str)
+def test_poses_against_oracle(robot, counts, gpu, oracle_robots):
+    """Pose checks answer lane by lane, so lanes retire one by one while the
+    balls of the gate pass stand: paths (checked by balls over the wave) and
+    samples (checked pose by pose), in whole waves and a ragged one."""
+    from prrtc_amd.robots import limits
+    R = oracle_robots[robot]
+    sc = _scene(counts, 7 + sum(counts))
+    lo, span = limits(robot)
+    rng = np.random.default_rng(13)
+    few = sum(counts) > 1000
+    samples = (lo + span * rng.random((70 if few else 301, len(lo)), dtype=F32)).astype(F32)
+    u = rng.normal(size=(2 if few else 5, 1, len(lo)))
+    u /= np.linalg.norm(u, axis=2, keepdims=True)
+    paths = samples[:len(u), None, :] + np.linspace(0, 0.8, 64)[None, :, None] * u
+    for q in (samples, paths.reshape(-1, len(lo)).astype(F32)[:-7]):
+        got = gpu.check_poses(robot, sc, q)
+        want, margin = R.check(sc, q, margin=True)
+        assert np.all(margin[got != want] < NEAR)
+
+
+@pytest.mark.gpu
 def test_pose_that_is_no_number(gpu, oracle_robots):
     """A cuboid's test takes a NaN position for a hit (utils.cuh:158-175: the
     NaN is dropped by max(0, .)), a sphere's for none; neither may be lost
