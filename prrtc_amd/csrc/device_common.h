@@ -69,9 +69,16 @@ struct Share {
     int part = 0, shift = 0;
 };
 
-// LDS float4 of a staged scene: its tables (scene_f4) and the balls, at most
-// one per two float4 of tables (every obstacle but a sphere has two or more).
-__host__ __device__ constexpr int scene_lds_f4(int scene_f4) { return scene_f4 + scene_f4 / 2; }
+// LDS float4 of a staged scene: its tables and a ball for every obstacle that
+// is not a sphere.  Where the host sees only a device copy (scene_f4 float4 of
+// tables): the most it can be, one ball per two float4 of tables.  What a
+// workgroup asks for and does not use costs resident waves: 65536 Baxter poses
+// against 4096 spheres, asked for 96 KiB and for the 64 they need, 10.5 and 5.8
+// ms; 1024 boxes, 96 and 80 KiB, 5.1 and 2.8 ms.
+__host__ __device__ constexpr int scene_lds_f4(int n_sph, int n_cap, int n_zcap, int n_cub, int n_zcub) {
+    return n_sph + 3 * (n_cap + n_zcap) + 5 * (n_cub + n_zcub);
+}
+__host__ __device__ constexpr int scene_lds_f4_most(int scene_f4) { return scene_f4 + scene_f4 / 2; }
 
 // Read a packed scene's header.  `cap_f4` is the payload size the host
 // allocated; a header that does not fit it (or is inconsistent) is read as an
@@ -100,7 +107,7 @@ __device__ __forceinline__ float capsule_ball_radius(float vx, float vy, float v
 }
 
 // Copy a packed scene's payload into LDS and append the balls
-// (scene_lds_f4(cap_f4) float4 in all); every lane of the workgroup helps.
+// (scene_lds_f4 of it in all); every lane of the workgroup helps.
 __device__ inline void stage_scene(const float *packed, int cap_f4, float4 *lds, SceneHeader &h) {
 #pragma clang fp contract(off)
     read_header(packed, cap_f4, h);
@@ -676,7 +683,7 @@ struct SpreadCtx : CheckCtx {
 struct SphereRobot {     // Robots.hh:190-237; fkcc<Sphere>, utils.cuh:330-334
     static constexpr int DOF = 3;
     static constexpr int NSPHERES = 1;
-    static constexpr float kSpread = 2.0f;   // in its cube of side 10
+    static constexpr float kSpread = 4.0f;   // its positions lie in a cube of side 10
     __host__ __device__ static constexpr float lower(int) { return -5.0f; }
     __host__ __device__ static constexpr float span(int) { return 10.0f; }
     template <class Ctx>

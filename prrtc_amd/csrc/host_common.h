@@ -75,6 +75,7 @@ int robot_dof(int robot);
 int robot_num_spheres(int robot);
 bool scene_valid(const prrtc_scene *s);
 size_t scene_packed_floats(const prrtc_scene *s);
+int scene_lds_f4(const prrtc_scene *s);
 void scene_pack(const prrtc_scene *s, float *out);
 int num_cus();
 

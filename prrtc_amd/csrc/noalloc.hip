@@ -131,7 +131,7 @@ int solve_noalloc(const HostProblem &hp, prrtc_result *out, float *path, int pat
     const int64_t tk = now_ns();
     launch_plan_init(hp.robot, d_desc, d_state, nullptr, 1, s);
     launch_plan_slice(hp.robot, d_desc, d_state, d_ctrl, d_paths, plan_grid(hp.robot, waves, hp.st->num_new_configs),
-                      waves, scene_lds_f4((L.scene_floats - 8) / 4), L.max_ext, s);
+                      waves, L.lds_f4, L.max_ext, s);
     PlanState ps;
     PRRTC_HIP(hipMemcpyAsync(&ps, d_state, sizeof ps, hipMemcpyDeviceToHost, s));
     PRRTC_HIP(hipStreamSynchronize(s));

@@ -1106,6 +1106,7 @@ BlockLayout block_layout(const HostProblem &hp) {
     const int nnc = hp.st->num_new_configs;
     BlockLayout L;
     L.scene_floats = (int)scene_packed_floats(hp.scene);
+    L.lds_f4 = scene_lds_f4(hp.scene);
     // storage rounded up to whole 1024-node scan chunks (16-byte aligned SoA
     // columns, the nearest-node scan reads whole chunks); the node limit
     // stays max_samples
@@ -1418,7 +1419,7 @@ static void start_group(GroupRun &gr, int path_cap) {
     std::vector<size_t> o_block(P);
     int lds_f4 = 0, ext_all = 0;
     for (int i = 0; i < P; i++) {
-        lds_f4 = std::max(lds_f4, scene_lds_f4((lay[i].scene_floats - 8) / 4));
+        lds_f4 = std::max(lds_f4, lay[i].lds_f4);
         ext_all = std::max(ext_all, lay[i].max_ext);
         o_block[i] = dl.take(lay[i].bytes);
     }

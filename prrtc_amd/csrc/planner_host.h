@@ -27,6 +27,7 @@ struct BlockLayout {
     size_t upload_bytes = 0;    // scene + init, contiguous at the block start
     size_t bytes = 0;           // whole block (256-byte multiple)
     int cap = 0, max_ext = 0, scene_floats = 0;
+    int lds_f4 = 0;             // float4 of LDS the staged scene takes
 };
 
 // Internal robot id of a launch whose problems have different robots (one

@@ -367,7 +367,7 @@ void ServerImpl::launch(RobotClass &c) {
         // waiting behind the young requests of a busy server
         if (!rq->stop_reason && (any_stopped || rq->round >= cfg.young_rounds))
             c.h_mask[2 * W + (e >> 6)] |= 1ull << (e & 63);
-        lds_f4 = std::max(lds_f4, scene_lds_f4((rq->lay.scene_floats - 8) / 4));
+        lds_f4 = std::max(lds_f4, rq->lay.lds_f4);
         ext = std::max(ext, rq->lay.max_ext);
         max_nnc = std::max(max_nnc, rq->st.num_new_configs);
         slots += rq->st.num_new_configs;

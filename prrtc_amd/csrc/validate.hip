@@ -170,6 +170,10 @@ size_t scene_packed_floats(const prrtc_scene *s) {
                                             s->n_z_cuboids);
 }
 
+int scene_lds_f4(const prrtc_scene *s) {
+    return scene_lds_f4(s->n_spheres, s->n_capsules, s->n_z_capsules, s->n_cuboids, s->n_z_cuboids);
+}
+
 void scene_pack(const prrtc_scene *s, float *out) {
     const int nf4 = scene_payload_f4(s->n_spheres, s->n_capsules, s->n_z_capsules, s->n_cuboids, s->n_z_cuboids);
     int32_t hdr[8] = {s->n_spheres, s->n_capsules, s->n_z_capsules, s->n_cuboids, s->n_z_cuboids, nf4, 0, 0};
@@ -211,20 +215,20 @@ int num_cus() {
 }
 
 template <class... KArgs, class... Args>
-static void launch_scene_kernel(void (*k)(KArgs...), dim3 grid, size_t scene_f4, hipStream_t st, Args... args) {
-    hipLaunchKernelGGL(k, grid, dim3(kWave), scene_lds_f4((int)scene_f4) * sizeof(float4), st, args...);
+static void launch_scene_kernel(void (*k)(KArgs...), dim3 grid, int lds_f4, hipStream_t st, Args... args) {
+    hipLaunchKernelGGL(k, grid, dim3(kWave), lds_f4 * sizeof(float4), st, args...);
     PRRTC_HIP(hipGetLastError());
 }
 
 template <class Robot>
-static void launch_validate(const float *d_scene, size_t scene_f4, const float *d_edges, int n, int g,
+static void launch_validate(const float *d_scene, size_t scene_f4, int lds_f4, const float *d_edges, int n, int g,
                             uint8_t *d_out, hipStream_t st) {
     // three workgroups for each of the eight waves a CU holds: edges take
     // uneven time, and the last ones even out; each workgroup stages the
     // scene, so many more would cost.  Against two: 10k Fetch edges 82 -> 79
     // us (139 -> 131 on another scene), 30k Baxter edges 260 -> 249 us.
     const int grid = std::max(1, std::min(n, num_cus() * 24));
-    launch_scene_kernel(k_validate_edges<Robot>, dim3(grid), scene_f4, st, d_scene, (int)scene_f4, d_edges,
+    launch_scene_kernel(k_validate_edges<Robot>, dim3(grid), lds_f4, st, d_scene, (int)scene_f4, d_edges,
                         n, g, d_out);
 }
 
@@ -253,16 +257,18 @@ static bool poses_apart(const float *poses, int n, int dof, float apart) {
 // pose by pose (SpreadCtx), since balls around them rule out little and cost
 // their own forming and a branch per gate and obstacle.  kSpread is the length
 // of a 64-pose path at which both take the same time: Panda 2 to 2.5, Fetch
-// 1.5 to 2, Baxter 4 to 5, UR5 3 to 5, over scenes of 12 to 4096 obstacles.
+// 1.5 to 2, Baxter 4 to 5, UR5 3 to 5, over scenes of 12 to 4096 obstacles
+// (the point robot 4, in metres).
 // 4096 uniform poses by balls and pose by pose: Panda, 72 obstacles 207 and 157
 // us, 1000 spheres 1182 and 860; Baxter, 32 boxes 73 and 50 us, 1000 spheres
 // 1084 and 648.  64 paths of 0.5 rad: Panda, 72 obstacles 26 and 48 us, 1000
-// spheres 73 and 236.
+// spheres 73 and 236.  65536 uniform positions of the point robot among 1000
+// spheres: 149 and 32 us.
 template <class Robot>
-static void launch_check(const float *d_scene, size_t scene_f4, const float *d_poses, int n, bool apart, uint8_t *d_out,
-                         hipStream_t st) {
+static void launch_check(const float *d_scene, size_t scene_f4, int lds_f4, const float *d_poses, int n, bool apart,
+                         uint8_t *d_out, hipStream_t st) {
     const int blocks = std::max(1, std::min((n + kWave - 1) / kWave, num_cus() * 16));
-    launch_scene_kernel(apart ? k_check_poses<Robot, SpreadCtx> : k_check_poses<Robot, CheckCtx>, dim3(blocks), scene_f4,
+    launch_scene_kernel(apart ? k_check_poses<Robot, SpreadCtx> : k_check_poses<Robot, CheckCtx>, dim3(blocks), lds_f4,
                         st, d_scene, (int)scene_f4, d_poses, n, d_out);
 }
 
@@ -478,7 +484,8 @@ int prrtc_check_poses(int robot, const prrtc_scene *scene, const float *poses, i
                                                     float spread = 0.0f;
                                                     PRRTC_DISPATCH(robot, spread_of, spread);
                                                     const bool apart = poses_apart(poses, n, D, spread);
-                                                    PRRTC_DISPATCH(robot, launch_check, ds, f4, dq, n, apart, dout, st);
+                                                    PRRTC_DISPATCH(robot, launch_check, ds, f4, scene_lds_f4(scene), dq, n, apart,
+                                                                   dout, st);
                                                 })
                                  : all_finite(poses, (size_t)n * D);
         if (!finite) {
@@ -506,8 +513,8 @@ int prrtc_validate_edges(int robot, const prrtc_scene *scene, const float *edges
         const bool fits = scene_fits(f4);
         const bool finite = fits ? verdict_call(scene, edges, (size_t)n * 2 * D, n, out_free,
                                                 [&](const float *ds, const float *de, uint8_t *dout, hipStream_t st) {
-                                                    PRRTC_DISPATCH(robot, launch_validate, ds, f4, de, n, granularity,
-                                                                   dout, st);
+                                                    PRRTC_DISPATCH(robot, launch_validate, ds, f4, scene_lds_f4(scene), de, n,
+                                                                   granularity, dout, st);
                                                 })
                                  : all_finite(edges, (size_t)n * 2 * D);
         if (!finite) {
@@ -536,8 +543,9 @@ int prrtc_validate_edges_async(int robot, const float *d_scene, size_t scene_flo
             set_error("prrtc_validate_edges_async: scene tables exceed %zu bytes", kMaxLdsScene);
             return PRRTC_EINVAL;
         }
-        PRRTC_DISPATCH(robot, launch_validate, d_scene, (scene_floats - 8) / 4, d_edges, n, granularity, d_out_free,
-                       (hipStream_t)stream);
+        const size_t f4 = (scene_floats - 8) / 4;
+        PRRTC_DISPATCH(robot, launch_validate, d_scene, f4, scene_lds_f4_most((int)f4), d_edges, n, granularity,
+                       d_out_free, (hipStream_t)stream);
         return PRRTC_OK;
     });
 }
