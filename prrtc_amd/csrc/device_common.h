@@ -93,17 +93,20 @@ __device__ inline void read_header(const float *packed, int cap_f4, SceneHeader 
     if (!ok) h = SceneHeader{0, 0, 0, 0, 0, 0, 0, 0};
 }
 
-__device__ __forceinline__ float sq3(float dx, float dy, float dz) {
+__host__ __device__ __forceinline__ float sq3(float dx, float dy, float dz) {
 #pragma clang fp contract(off)
     return fmaf(dx, dx, fmaf(dy, dy, dz * dz));
 }
 
-// Radius of the ball about a segment's midpoint that holds the capsule:
-// |v|/2 + r, padded by 2^-16 relative and 1 mm absolute.  The pad covers the
-// rounding of sqrtf and of the tests it replaces many times over.
-__device__ __forceinline__ float capsule_ball_radius(float vx, float vy, float vz, float r) {
+// Ball about a segment's midpoint that holds the capsule of rows (p, r) and
+// (v, .): radius |v|/2 + |r| (a test squares r + the sphere's radius, so a
+// negative one reaches as far), padded by 2^-16 relative and 1 mm absolute.  The
+// pad covers the rounding of sqrtf and of the tests it replaces many times
+// over.
+__host__ __device__ __forceinline__ float4 capsule_ball(const float4 &p, float vx, float vy, float vz) {
 #pragma clang fp contract(off)
-    return fmaf(0.5f * sqrtf(sq3(vx, vy, vz)) + r, 1.0f + 0x1p-16f, 1e-3f);
+    return make_float4(fmaf(0.5f, vx, p.x), fmaf(0.5f, vy, p.y), fmaf(0.5f, vz, p.z),
+                       fmaf(0.5f * sqrtf(sq3(vx, vy, vz)) + fabsf(p.w), 1.0f + 0x1p-16f, 1e-3f));
 }
 
 // Copy a packed scene's payload into LDS and append the balls
@@ -121,8 +124,7 @@ __device__ inline void stage_scene(const float *packed, int cap_f4, float4 *lds,
             const float4 p = cap[2 * i];
             float4 v = cap[2 * i + 1];
             if (i >= h.n_cap) v.x = v.y = 0.0f;   // a z-capsule's test reads v.z alone
-            b = make_float4(fmaf(0.5f, v.x, p.x), fmaf(0.5f, v.y, p.y), fmaf(0.5f, v.z, p.z),
-                            capsule_ball_radius(v.x, v.y, v.z, p.w));
+            b = capsule_ball(p, v.x, v.y, v.z);
         } else {
             const float4 *row = cub + 4 * (i - n_caps);
             b = row[0];
@@ -199,6 +201,15 @@ struct WaveBall {
     float x, y, z, r;
 };
 
+__host__ __device__ __forceinline__ float padded_root(float d2) {
+#pragma clang fp contract(off)
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_sqrtf(d2) * (1.0f + 0x1p-16f);
+#else
+    return sqrtf(d2) * (1.0f + 0x1p-16f);
+#endif
+}
+
 // Centre of the ball: midway between the first and the last live lane's
 // point (the ends of the wave's stretch of the path).
 __device__ __forceinline__ WaveBall ball_centre(float x, float y, float z, uint64_t live) {
@@ -216,7 +227,7 @@ __device__ __forceinline__ WaveBall ball_centre(float x, float y, float z, uint6
 __device__ __forceinline__ float ball_radius(float d2, bool live) {
 #pragma clang fp contract(off)
     const uint32_t m = wave_max(live ? (uint32_t)__float_as_int(d2) : 0u);
-    return __builtin_amdgcn_sqrtf(__int_as_float((int)m)) * (1.0f + 0x1p-16f);
+    return padded_root(__int_as_float((int)m));
 }
 
 // Point (x, y, z) of every live lane in one ball (`live`: the ballot of the
@@ -228,6 +239,11 @@ __device__ __forceinline__ WaveBall wave_ball(float x, float y, float z, bool on
     return c;
 }
 
+__host__ __device__ __forceinline__ float sphere_ball_radius(float r) {
+#pragma clang fp contract(off)
+    return fmaf(fabsf(r), 1.0f + 0x1p-16f, 1e-3f);
+}
+
 // One obstacle's ball on each lane: obstacle i of the scene.  A sphere's is
 // padded like the others (2^-16 relative, 1 mm).
 template <bool LOCAL>
@@ -235,7 +251,7 @@ __device__ __forceinline__ float4 obstacle_ball(const Obstacles &o, int i) {
 #pragma clang fp contract(off)
     const bool s = i < o.n_sph;
     float4 b = ld_obs<LOCAL>(s ? o.sph + i : o.ball + (i - o.n_sph));
-    if (s) b.w = fmaf(fabsf(b.w), 1.0f + 0x1p-16f, 1e-3f);
+    if (s) b.w = sphere_ball_radius(b.w);
     return b;
 }
 
@@ -243,7 +259,7 @@ __device__ __forceinline__ float4 obstacle_ball(const Obstacles &o, int i) {
 // obstacle ball `b`.  Both radii are padded, so an obstacle out of reach is
 // at least about 1 mm from every live lane's sphere: its exact test would be
 // positive, and skipping it cannot change a verdict.  NaN counts as in reach.
-__device__ __forceinline__ bool in_reach(const float4 &b, const WaveBall &c, float reach) {
+__host__ __device__ __forceinline__ bool in_reach(const float4 &b, const WaveBall &c, float reach) {
 #pragma clang fp contract(off)
     const float rb = reach + b.w;
     return !(sq3(b.x - c.x, b.y - c.y, b.z - c.z) > rb * rb);
@@ -255,12 +271,12 @@ __device__ __forceinline__ bool in_reach(const float4 &b, const WaveBall &c, flo
 // fixed association (and contraction is off), so the CPU oracle can reproduce
 // each verdict bit for bit in its "fused" mode.
 
-__device__ __forceinline__ float sphere_test(const float4 &s, float x, float y, float z, float r) {   // utils.cuh:58-81
+__host__ __device__ __forceinline__ float sphere_test(const float4 &s, float x, float y, float z, float r) {   // utils.cuh:58-81
 #pragma clang fp contract(off)
     const float rs = s.w + r;
     return fmaf(-rs, rs, sq3(s.x - x, s.y - y, s.z - z));
 }
-__device__ __forceinline__ float capsule_test(const float4 &p, const float4 &v, float x, float y, float z,
+__host__ __device__ __forceinline__ float capsule_test(const float4 &p, const float4 &v, float x, float y, float z,
                                               float r) {                                                // utils.cuh:113-126
 #pragma clang fp contract(off)
     const float dot = fmaf(x - p.x, v.x, fmaf(y - p.y, v.y, (z - p.z) * v.z));
@@ -268,7 +284,7 @@ __device__ __forceinline__ float capsule_test(const float4 &p, const float4 &v, 
     const float rs = r + p.w;
     return fmaf(-rs, rs, sq3(x - fmaf(v.x, cdf, p.x), y - fmaf(v.y, cdf, p.y), z - fmaf(v.z, cdf, p.z)));
 }
-__device__ __forceinline__ float z_capsule_test(const float4 &p, const float4 &v, float x, float y, float z,
+__host__ __device__ __forceinline__ float z_capsule_test(const float4 &p, const float4 &v, float x, float y, float z,
                                                 float r) {                                              // utils.cuh:135-148
 #pragma clang fp contract(off)
     const float dot = (z - p.z) * v.z;
@@ -276,7 +292,7 @@ __device__ __forceinline__ float z_capsule_test(const float4 &p, const float4 &v
     const float rs = r + p.w;
     return fmaf(-rs, rs, sq3(x - p.x, y - p.y, z - fmaf(v.z, cdf, p.z)));
 }
-__device__ __forceinline__ float cuboid_test(const float4 &c, const float4 &a1, const float4 &a2, const float4 &a3,
+__host__ __device__ __forceinline__ float cuboid_test(const float4 &c, const float4 &a1, const float4 &a2, const float4 &a3,
                                              float x, float y, float z, float r) {                      // utils.cuh:158-175
 #pragma clang fp contract(off)
     const float xs = x - c.x, ys = y - c.y, zs = z - c.z;
@@ -285,7 +301,7 @@ __device__ __forceinline__ float cuboid_test(const float4 &c, const float4 &a1, 
     const float d3 = fmaxf(0.0f, fabsf(fmaf(a3.x, xs, fmaf(a3.y, ys, a3.z * zs))) - a2.w);
     return fmaf(-r, r, sq3(d1, d2, d3));
 }
-__device__ __forceinline__ float z_cuboid_test(const float4 &c, const float4 &a1, const float4 &a2, float x, float y,
+__host__ __device__ __forceinline__ float z_cuboid_test(const float4 &c, const float4 &a1, const float4 &a2, float x, float y,
                                                float z, float r) {                                      // utils.cuh:184-201
 #pragma clang fp contract(off)
     const float xs = x - c.x, ys = y - c.y, zs = z - c.z;

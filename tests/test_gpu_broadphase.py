@@ -77,6 +77,30 @@ def test_poses_against_oracle(robot, counts, gpu, oracle_robots):
 
 
 @pytest.mark.gpu
+def test_negative_radius(gpu, oracle_robots):
+    """Obstacles of negative radius reach as far as the tests say, which square
+    the sum of the radii: bit for bit against the oracle on the point robot,
+    whose arithmetic both share."""
+    from oracle import oracle
+    from prrtc_amd import scenes as S
+    R = oracle_robots["sphere"]
+    rng = np.random.default_rng(4)
+    sc = S.Scene.build([S.sphere((-2, 0, 0), -1.9)], [S.cylinder_center((2, 1, 0), (0.3, 1, 2), -2.1, 0.5)],
+                       [S.cylinder_center((0, -3, 1), (0, 0, 0), -2.3, 0.4)])
+    a = rng.uniform(-5, 5, (4000, 3)).astype(F32)
+    edges = np.stack([a, a + rng.normal(size=a.shape).astype(F32) * F32(0.2)], 1)
+    oracle.set_fused(True)
+    try:
+        want = R.validate_edges(sc, edges, 16)
+        poses = R.check(sc, a)
+    finally:
+        oracle.set_fused(False)
+    assert 0.1 < want.mean() < 0.9
+    assert np.array_equal(gpu.validate_edges("sphere", sc, edges, 16), want)
+    assert np.array_equal(gpu.check_poses("sphere", sc, a), poses)
+
+
+@pytest.mark.gpu
 def test_pose_that_is_no_number(gpu, oracle_robots):
     """A cuboid's test takes a NaN position for a hit (utils.cuh:158-175: the
     NaN is dropped by max(0, .)), a sphere's for none; neither may be lost

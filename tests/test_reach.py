@@ -20,3 +20,18 @@ def reach(tmp_path_factory):
 def test_scene_lds(reach):
     """A workgroup asks for the LDS its scene takes and no more."""
     assert reach("lds").returncode == 0
+
+
+@pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
+def test_out_of_reach_hits_nothing(reach, sign):
+    """An obstacle of each kind brought along the tightest direction to the
+    first place where its ball is out of the wave's reach: every exact test is
+    positive there, and the surfaces keep the pads (1 mm, and half of 2^-16).  A sphere or
+    capsule of negative radius reaches as far as one of the positive (the tests
+    square the sum of the radii)."""
+    res = reach("reach", "-2", "0.5", str(sign))
+    assert res.returncode == 0, res.stdout
+    kinds = [line.split() for line in res.stdout.splitlines()]
+    assert len(kinds) == 5
+    for kind, used, spare in kinds:
+        assert int(used) == 4000 and float(spare) >= 0, kind
