@@ -85,8 +85,8 @@ def test_negative_radius(gpu, oracle_robots):
     from prrtc_amd import scenes as S
     R = oracle_robots["sphere"]
     rng = np.random.default_rng(4)
-    sc = S.Scene.build([S.sphere((-2, 0, 0), -1.9)], [S.cylinder_center((2, 1, 0), (0.3, 1, 2), -2.1, 0.5)],
-                       [S.cylinder_center((0, -3, 1), (0, 0, 0), -2.3, 0.4)])
+    sc = S.Scene.build([S.sphere((-2, 0, 0), -3.4)], [S.cylinder_center((2, 1, 0), (0.3, 1, 2), -3.1, 0.5)],
+                       [S.cylinder_center((0, -3, 1), (0, 0, 0), -3.3, 0.4)])
     a = rng.uniform(-5, 5, (4000, 3)).astype(F32)
     edges = np.stack([a, a + rng.normal(size=a.shape).astype(F32) * F32(0.2)], 1)
     oracle.set_fused(True)
