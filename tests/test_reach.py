@@ -22,14 +22,15 @@ def test_scene_lds(reach):
     assert reach("lds").returncode == 0
 
 
-@pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
-def test_out_of_reach_hits_nothing(reach, sign):
+@pytest.mark.parametrize("lo, hi, sign", [(-2, 0.5, 1), (-2, 0.5, -1), (2, 4, 1), (5, 7, 1)])
+def test_out_of_reach_hits_nothing(reach, lo, hi, sign):
     """An obstacle of each kind brought along the tightest direction to the
     first place where its ball is out of the wave's reach: every exact test is
     positive there, and the surfaces keep the pads (1 mm, and half of 2^-16).  A sphere or
     capsule of negative radius reaches as far as one of the positive (the tests
-    square the sum of the radii)."""
-    res = reach("reach", "-2", "0.5", str(sign))
+    square the sum of the radii), and positions far from the origin (up to 10^7
+    m) are rounded to more than the 1 mm."""
+    res = reach("reach", str(lo), str(hi), str(sign))
     assert res.returncode == 0, res.stdout
     kinds = [line.split() for line in res.stdout.splitlines()]
     assert len(kinds) == 5
