@@ -101,15 +101,16 @@ __host__ __device__ __forceinline__ float sq3(float dx, float dy, float dz) {
 // Ball about a segment's midpoint that holds the capsule of rows (p, r) and
 // (v, .): radius |v|/2 + |r| (a test squares r + the sphere's radius, so a
 // negative one reaches as far), padded by 2^-16 relative, 1 mm absolute and
-// 2^-20 of the coordinates.  The pads cover the rounding of sqrtf, of the
-// midpoint and of the tests they replace many times over (the midpoint and a
-// test's nearest point on the segment are rounded to 2^-24 of the
+// 2^-20 of the midpoint's coordinates.  The pads cover the rounding of sqrtf,
+// of the midpoint and of the tests they replace many times over (the midpoint
+// and a test's nearest point on the segment are rounded to 2^-24 of their
 // coordinates, more than 1 mm beyond 16 km).
 __host__ __device__ __forceinline__ float4 capsule_ball(const float4 &p, float vx, float vy, float vz) {
 #pragma clang fp contract(off)
-    const float far = fabsf(p.x) + fabsf(p.y) + fabsf(p.z) + fabsf(vx) + fabsf(vy) + fabsf(vz);
-    return make_float4(fmaf(0.5f, vx, p.x), fmaf(0.5f, vy, p.y), fmaf(0.5f, vz, p.z),
-                       fmaf(0.5f * sqrtf(sq3(vx, vy, vz)) + fabsf(p.w), 1.0f + 0x1p-16f, fmaf(0x1p-20f, far, 1e-3f)));
+    const float x = fmaf(0.5f, vx, p.x), y = fmaf(0.5f, vy, p.y), z = fmaf(0.5f, vz, p.z);
+    const float far = fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z));
+    return make_float4(x, y, z, fmaf(0.5f * sqrtf(sq3(vx, vy, vz)) + fabsf(p.w), 1.0f + 0x1p-16f,
+                                     fmaf(0x1p-20f, far, 1e-3f)));
 }
 
 // Copy a packed scene's payload into LDS and append the balls
