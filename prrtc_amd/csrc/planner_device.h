@@ -172,9 +172,13 @@ __device__ __forceinline__ int wave_atomic_add(int *p, int v) {
 // 79.5 -> 64.5 ms, an uneven batch of 128 problems 156 -> 125 ms, one Panda
 // solve 195 -> 169 us.
 // Wait until this wave's stores have reached L2, and order them before what
-// the workgroup's other waves, or this wave's other lanes, do next.
+// the workgroup's other waves, or this wave's other lanes, do next.  The wait
+// is an asm statement that touches memory, so no store written before the call
+// can be placed after it: the leader's releasing count waits only for its own
+// wave's stores, and this wait is what puts the other waves' in L2 before it.
+// (In flight on gfx950 are loads and stores alike: vmcnt counts both.)
 __device__ __forceinline__ void stores_done() {
-    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0), the other counters as they are
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
 }
 
