@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "robots/baxter.gen.h"
@@ -553,11 +554,14 @@ __device__ __forceinline__ bool self_hit(float ax, float ay, float az, float bx,
 // problems 219 -> 163 ms, a served burst 105 -> 63 ms.)  near[w] gets the
 // groups 64 w .. 64 w + 63 that do, of those whose number is sh.part mod
 // 2^sh.shift (the wave's own).
-constexpr int kSelfWords = 6;   // up to 384 groups
+// Words of 64 for the robot that has the most groups; a robot's check touches
+// the words of its own only.
+constexpr int kSelfWords = (std::max({gen::panda::SELF_GROUPS, gen::fetch::SELF_GROUPS, gen::baxter::SELF_GROUPS,
+                                      gen::ur5::SELF_GROUPS}) + 63) / 64;
 
 template <int NS>
 __device__ __forceinline__ void self_groups_own(Share sh, uint64_t (&near)[kSelfWords]) {
-    static_assert(NS <= 64 * kSelfWords, "groups fit the mask");
+    static_assert(NS <= 64 * kSelfWords, "a robot is missing in kSelfWords");
     const int lane = threadIdx.x & (kWave - 1);
     const uint64_t own = ballot((lane & ((1 << sh.shift) - 1)) == sh.part);   // 64 is a multiple of 2^shift
 #pragma unroll
@@ -568,7 +572,7 @@ template <int NS>
 __device__ __forceinline__ void self_groups_near(Share sh, const uint32_t *pairs, const WaveBall &balls,
                                                  uint64_t (&near)[kSelfWords]) {
 #pragma clang fp contract(off)
-    static_assert(NS <= 64 * kSelfWords, "groups fit the mask");
+    static_assert(NS <= 64 * kSelfWords, "a robot is missing in kSelfWords");
     const int lane = threadIdx.x & (kWave - 1);
     const bool own = (lane & ((1 << sh.shift) - 1)) == sh.part;
     auto from = [](float v, uint32_t k) {

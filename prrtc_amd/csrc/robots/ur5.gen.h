@@ -4,6 +4,7 @@
 namespace prrtc::gen::ur5 {
 constexpr int DOF = 6;
 constexpr int NSPHERES = 29;
+constexpr int SELF_GROUPS = 33;
 __device__ __host__ constexpr float lower(int i) { constexpr float v[] = {-3.1415927410125732f, -3.1415927410125732f, -3.1415927410125732f, -3.1415927410125732f, -3.1415927410125732f, -3.1415927410125732f}; return v[i]; }
 __device__ __host__ constexpr float span(int i) { constexpr float v[] = {6.2831854820251465f, 3.1415927410125732f, 6.2831854820251465f, 6.2831854820251465f, 6.2831854820251465f, 6.2831854820251465f}; return v[i]; }
 

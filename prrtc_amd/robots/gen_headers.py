@@ -116,6 +116,7 @@ def gen_robot_from(m: dict) -> str:
     w(f"namespace prrtc::gen::{name} {{")
     w(f"constexpr int DOF = {dof};")
     w(f"constexpr int NSPHERES = {len(sph)};")
+    w(f"constexpr int SELF_GROUPS = {sum(kind == 'self' for kind, _ in m['order'])};")
     w("__device__ __host__ constexpr float lower(int i) { constexpr float v[] = {" +
       ", ".join(flit(x) for x in m["lower"]) + "}; return v[i]; }")
     w("__device__ __host__ constexpr float span(int i) { constexpr float v[] = {" +

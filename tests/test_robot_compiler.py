@@ -232,3 +232,34 @@ def test_ur5_oracle_verdicts_brute_force(oracle_robots):
     far = np.minimum(np.abs(d).min(axis=(1, 2)), np.abs(dp).min(axis=1)) > 1e-5
     assert far.sum() > 300 and 0.1 < brute_free.mean() < 0.9, (far.sum(), brute_free.mean())
     assert np.array_equal(free[far].astype(bool), brute_free[far])
+
+
+def test_more_self_groups_than_any_robot(tmp_path):
+    """A robot may have any number of self-collision groups: Baxter's table
+    with its groups listed three times (1,065) through the generator, and its
+    check instantiated for edges."""
+    import shutil
+    import subprocess
+    from prrtc_amd.build import FLAGS, HIPCC
+    from prrtc_amd.robots import gen_headers, load_model
+    m = load_model("baxter")
+    n = len(m["self_checks"])
+    selfs = [o for o in m["order"] if o[0] == "self"]
+    many = dict(m, self_checks=m["self_checks"] * 3,
+                order=[*m["order"], *([k, i + n] for k, i in selfs), *([k, i + 2 * n] for k, i in selfs)])
+    csrc = tmp_path / "prrtc_amd" / "csrc"
+    shutil.copytree(os.path.join(ROOT, "prrtc_amd", "csrc"), csrc)
+    shutil.copytree(os.path.join(ROOT, "include"), tmp_path / "include")
+    (csrc / "robots" / "baxter.gen.h").write_text(gen_headers.gen_robot_from(many))
+    (csrc / "many.hip").write_text("""
+#include "host_common.h"
+using namespace prrtc;
+__global__ void many(const float *q, int *hit) {
+    CheckCtx ctx{};
+    BaxterRobot::check(q, ctx);
+    hit[threadIdx.x] = ctx.coll;
+}
+""")
+    res = subprocess.run([HIPCC, *FLAGS, "--offload-device-only", "-fsyntax-only", str(csrc / "many.hip")],
+                         capture_output=True, text=True, timeout=120)
+    assert res.returncode == 0, res.stderr[-2000:]
