@@ -13,21 +13,11 @@
 
 #include "../../include/prrtc.h"
 #include "device_common.h"
+#include "host_call.h"
 
 namespace prrtc {
 
 void set_error(const char *fmt, ...);
-
-struct HipError {
-    hipError_t code;
-    const char *where;
-};
-
-#define PRRTC_HIP(call)                                                   \
-    do {                                                                  \
-        hipError_t _e = (call);                                           \
-        if (_e != hipSuccess) throw ::prrtc::HipError{_e, #call};         \
-    } while (0)
 
 // Run `body`, turning exceptions into status codes and the thread's message.
 template <class F>

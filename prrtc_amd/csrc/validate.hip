@@ -314,46 +314,6 @@ static bool copy_finite(float *dst, const float *src, size_t n) {
     return bad == 0;
 }
 
-// Device buffer, pinned staging and stream of a thread's host-buffer calls
-// (check_poses, validate_edges), kept between calls: three device
-// allocations and frees and three blocking copies were 110 of the 150 us of
-// a 4096-pose check.  At most kMost bytes of each, released when the thread
-// ends; a larger call brings its own (verdict_call).  Every call waits for
-// its own work, so a buffer is never in use when the thread's next call takes
-// it.
-struct HostCall {
-    static constexpr size_t kMost = 16u << 20;
-    char *dev = nullptr, *host = nullptr;
-    size_t bytes = 0;   // of each
-    hipStream_t stream = nullptr;
-    int device = -1;   // of the buffers and the stream
-
-    void release() {
-        if (dev) (void)hipFree(dev);
-        if (host) (void)hipHostFree(host);
-        if (stream) (void)hipStreamDestroy(stream);
-        dev = host = nullptr;
-        bytes = 0;
-        stream = nullptr;
-        device = -1;
-    }
-    ~HostCall() { release(); }
-    // Both buffers of at least n <= kMost bytes on the thread's current device.
-    void need(size_t n) {
-        int cur = 0;
-        PRRTC_HIP(hipGetDevice(&cur));
-        if (cur != device || n > bytes) {
-            release();
-            const size_t size = std::min(kMost, n + n / 2 + 65536);
-            PRRTC_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-            PRRTC_HIP(hipMalloc(&dev, size));
-            PRRTC_HIP(hipHostMalloc(&host, size, hipHostMallocDefault));
-            bytes = size;
-            device = cur;
-        }
-    }
-};
-
 static HostCall &host_call() {
     static thread_local HostCall hc;
     return hc;
