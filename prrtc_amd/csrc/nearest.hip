@@ -186,15 +186,28 @@ template <int D>
 static void launch_nearest(const float *trees, int cap, int n, const float *queries, int qpt, int n_trees,
                            int waves, int *idx, float *dist2, hipStream_t s) {
     const int n_queries = n_trees * qpt;
-    // As many queries per workgroup as leave two workgroups for every CU:
-    // fewer would idle part of the chip for longer than the shared reads save.
-    auto fills = [&](int q) { return qpt >= q && (long long)n_trees * ((qpt + q - 1) / q) >= 2ll * num_cus(); };
+    // As many queries per workgroup as leave every CU two workgroups and a wave
+    // for each SIMD, two where D is 3 and the shared reads save least: fewer
+    // would idle part of the chip for longer than they save.  (64 trees of 50k
+    // nodes, 64 queries each, one wave, D 7 and 8: 193 and 220 us a query at a
+    // time; eight to a workgroup, half the SIMDs idle, 282 and 300; four, 174
+    // and 184.  D 3: 90 us; four to a workgroup 147.)
+    auto fills = [&](int q) {
+        const long long tiles = (long long)n_trees * ((qpt + q - 1) / q);
+        return qpt >= q && tiles >= 2ll * num_cus() && tiles * waves >= (D > 3 ? 4ll : 8ll) * num_cus();
+    };
     // (a query's coordinates take D scalar registers: 8 of 14 do not fit)
     if constexpr (D <= 8) {
         if (fills(8)) return launch_tile<D, 8>(trees, cap, n, queries, qpt, n_trees, waves, idx, dist2, s);
     }
     if (fills(4)) return launch_tile<D, 4>(trees, cap, n, queries, qpt, n_trees, waves, idx, dist2, s);
-    if (fills(2)) return launch_tile<D, 2>(trees, cap, n, queries, qpt, n_trees, waves, idx, dist2, s);
+    // A pair saves three of six reads a node where D is 3, which is no more
+    // than a half-empty pair or a one-wave workgroup costs: 256 trees of 50k
+    // nodes, 3 queries each, four waves, 32 us a query at a time, 36 in pairs;
+    // 64 trees, 64 queries, one wave, 90 and 102; 8 trees, 128 queries, four
+    // waves, 32 and 28.
+    if (fills(2) && (D > 3 || (qpt % 2 == 0 && waves > 1)))
+        return launch_tile<D, 2>(trees, cap, n, queries, qpt, n_trees, waves, idx, dist2, s);
     const int grid = std::max(1, std::min(n_queries, num_cus() * 64));
     hipLaunchKernelGGL(k_nearest<D>, dim3(grid), dim3(waves * kWave), 0, s, trees, cap, n, queries, qpt, n_queries,
                        idx, dist2);
