@@ -35,15 +35,6 @@ def test_commits_equal_the_oracle(nnc, dd, gpu, oracle_robots):
         oracle.set_fused(False)
 
 
-def test_chain_passes_shared_or_apart(gpu):
-    """Chain passes whose waves take poses of their own (the default) and
-    passes that share 64 poses give the same solves, bit for bit."""
-    import test_gpu_shapes as T
-    base = T.solve_digests()
-    assert T._child({"PRRTC_WIDE_FROM": "-1"}) == base
-    assert T._child({"PRRTC_WIDE_FROM": "2"}) == base
-
-
 @pytest.mark.parametrize("robot", ["fetch", "baxter"])
 def test_largest_scene_and_chains(robot, gpu):
     """The most LDS a planner workgroup can ask for: full obstacle tables (64

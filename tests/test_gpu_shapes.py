@@ -1,10 +1,10 @@
 """Pass shapes never change a result.  A planner task's waves either share
 a validation pass's 64 poses (splitting the obstacles) or take poses of
-their own; the library picks per robot and per task.  The same problems are
-solved here with the default shapes and in child processes with every
-connect-chain pass allowed to go wide (PRRTC_WIDE_FROM=0, Fetch included,
-whose default is never) and with steered edges kept on shared passes
-(PRRTC_WIDE_EDGE=0): every result and path must be bit for bit the same."""
+their own, as connect chains do from their first pass on.  The same problems
+are solved here so and in child processes with chain passes always shared
+(PRRTC_WIDE_FROM=-1), with the first two shared (2), and with steered edges
+kept on shared passes (PRRTC_WIDE_EDGE=0): every result and path must be bit
+for bit the same."""
 import hashlib
 import json
 import os
@@ -21,9 +21,8 @@ ROOT = os.path.dirname(HERE)
 
 
 def solve_digests():
-    """Fetch C2 problems (g 64, nnc 64: rounds leave CUs free, so chain
-    passes may go wide) and Panda C1 plans (g 128: steered edges of 128
-    poses), alone; one digest per solve."""
+    """Fetch C2 problems (g 64), Panda C1 plans (g 128: steered edges of 128
+    poses) and Baxter and UR5 problems, alone; one digest per solve."""
     import prrtc_amd as P
     from prrtc_amd import workloads
     P.load()
@@ -36,6 +35,8 @@ def solve_digests():
                dd_radius=4.0, dd_alpha=1e-4, dd_min_radius=1.0, max_samples=100000, max_iters=200)
     for i, p in enumerate(workloads.c1_problems(3, seed=1)):
         out.append(_digest(*P.solve("panda", p["start"], p["goals"], p["scene"], dict(pst, seed=i))))
+    for p in workloads.c3_problems(3, 0, 0, seed=0) + workloads.ur5_problems(3, seed=0):
+        out.append(_digest(*P.solve(p["robot"], p["start"], p["goals"], p["scene"], fst)))
     return out
 
 
@@ -60,8 +61,8 @@ def _child(env_extra):
 
 def test_pass_shapes_same_results(gpu):
     base = solve_digests()
-    assert len(base) == 9
-    for env_extra in ({"PRRTC_WIDE_FROM": "0"}, {"PRRTC_WIDE_EDGE": "0"}):
+    assert len(base) == 15
+    for env_extra in ({"PRRTC_WIDE_FROM": "-1"}, {"PRRTC_WIDE_FROM": "2"}, {"PRRTC_WIDE_EDGE": "0"}):
         got = _child(env_extra)
         bad = [i for i, (a, b) in enumerate(zip(base, got)) if a != b]
         assert not bad, f"{env_extra}: solves {bad} differ"
