@@ -1,5 +1,5 @@
 """Algorithmic work of collision checking, counted the way the reference
-executes it -- the denominator of the validation roofline.
+executes it: what the kernels' broad phase saves is counted too.
 
 For one pose the reference's fkcc<Robot> (src/planning/utils.cuh:336-33131)
 runs its straight-line FK and then, in check order, every link's gate
