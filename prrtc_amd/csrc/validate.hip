@@ -344,19 +344,19 @@ static bool verdict_call(const prrtc_scene *scene, const float *in, size_t n_flo
     HostCall &hc = host_call();
     hc.need(total);
     if (!copy_finite(reinterpret_cast<float *>(hc.host + scene_bytes), in, n_floats)) return false;
+    const hipStream_t s = nullptr;
     struct Drain {   // a call that fails half way leaves nothing queued on the buffers
-        hipStream_t s;
         bool done = false;
         ~Drain() {
-            if (!done) (void)hipStreamSynchronize(s);
+            if (!done) (void)hipStreamSynchronize(nullptr);
         }
-    } drain{hc.stream};
+    } drain;
     scene_pack(scene, reinterpret_cast<float *>(hc.host));
-    PRRTC_HIP(hipMemcpyAsync(hc.dev, hc.host, scene_bytes + sizeof(float) * n_floats, hipMemcpyHostToDevice, hc.stream));
+    PRRTC_HIP(hipMemcpyAsync(hc.dev, hc.host, scene_bytes + sizeof(float) * n_floats, hipMemcpyHostToDevice, s));
     launch(reinterpret_cast<const float *>(hc.dev), reinterpret_cast<const float *>(hc.dev + scene_bytes),
-           reinterpret_cast<uint8_t *>(hc.dev + up), hc.stream);
-    PRRTC_HIP(hipMemcpyAsync(hc.host + up, hc.dev + up, (size_t)n, hipMemcpyDeviceToHost, hc.stream));
-    PRRTC_HIP(hipStreamSynchronize(hc.stream));
+           reinterpret_cast<uint8_t *>(hc.dev + up), s);
+    PRRTC_HIP(hipMemcpyAsync(hc.host + up, hc.dev + up, (size_t)n, hipMemcpyDeviceToHost, s));
+    PRRTC_HIP(hipStreamSynchronize(s));
     drain.done = true;
     std::memcpy(out, hc.host + up, (size_t)n);
     return true;

@@ -1,6 +1,6 @@
 // HostCall (host_call.h) over a stand-in for the HIP runtime: live
-// allocations and streams are counted, freeing one that is not live fails the
-// run, and a device reset frees everything, the next allocations taking the
+// allocations are counted, freeing one that is not live fails the run, and a
+// device reset frees everything, the next allocations taking the
 // same addresses.  Run by tests/test_host_call.py.
 #include <cstdio>
 #include <cstdlib>
@@ -9,7 +9,7 @@
 #include "../../prrtc_amd/csrc/host_call.h"
 
 namespace {
-std::map<void *, unsigned long long> live;   // allocations and streams, by number
+std::map<void *, unsigned long long> live;   // allocations, by number
 unsigned long long last_id = 0;
 int device = 0, fail_after = -1;   // allocations until one fails (-1: none)
 alignas(256) char pool[64];
@@ -23,7 +23,7 @@ void check(bool ok, const char *what) {
 hipError_t take(void **p, int kind) {
     if (fail_after == 0) return hipErrorOutOfMemory;
     if (fail_after > 0) fail_after--;
-    for (int i = kind; i < 64; i += 4)   // the lowest free address of the kind
+    for (int i = kind; i < 64; i += 2)   // the lowest free address of the kind
         if (!live.count(pool + i)) {
             *p = pool + i;
             live[*p] = ++last_id;
@@ -44,8 +44,6 @@ hipError_t hipMalloc(void **p, size_t) { return take(p, 0); }
 hipError_t hipHostMalloc(void **p, size_t, unsigned) { return take(p, 1); }
 hipError_t hipFree(void *p) { return give(p, "freed device memory that is not live"); }
 hipError_t hipHostFree(void *p) { return give(p, "freed host memory that is not live"); }
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return take(reinterpret_cast<void **>(s), 2); }
-hipError_t hipStreamDestroy(hipStream_t s) { return give(s, "destroyed a stream that is not live"); }
 hipError_t hipPointerGetAttribute(void *out, hipPointer_attribute a, hipDeviceptr_t p) {
     check(a == HIP_POINTER_ATTRIBUTE_BUFFER_ID, "attribute");
     if (!live.count(p)) return hipErrorInvalidValue;
@@ -55,7 +53,7 @@ hipError_t hipPointerGetAttribute(void *out, hipPointer_attribute a, hipDevicept
 }
 
 static void usable(prrtc::HostCall &hc, size_t n) {
-    check(hc.bytes >= n && live.count(hc.dev) && live.count(hc.host) && live.count(hc.stream), "buffers are not live");
+    check(hc.bytes >= n && live.count(hc.dev) && live.count(hc.host), "buffers are not live");
     check(live[hc.dev] == hc.dev_id && live[hc.host] == hc.host_id, "buffers are someone else's");
 }
 
@@ -66,30 +64,29 @@ int main() {
         usable(hc, 1000);
         const unsigned long long id = hc.dev_id;
         hc.need(2000);
-        check(hc.dev_id == id && live.size() == 3, "a call that fits allocates nothing");
+        check(hc.dev_id == id && live.size() == 2, "a call that fits allocates nothing");
         hc.need(1 << 20);
         usable(hc, 1 << 20);
-        check(live.size() == 3, "the old buffers are freed");
+        check(live.size() == 2, "the old buffers are freed");
         device = 1;   // another device: buffers of its own
         hc.need(1000);
         usable(hc, 1000);
-        check(hc.device == 1 && live.size() == 3, "one set is kept");
+        check(hc.device == 1 && live.size() == 2, "one set is kept");
 
         live.clear();   // a device reset, and nothing since
         hc.need(1000);
         usable(hc, 1000);
-        check(live.size() == 3, "a new set after a reset");
+        check(live.size() == 2, "a new set after a reset");
         live.clear();   // a reset, and another owner at the same addresses
         void *d, *h;
-        hipStream_t s;
-        check(!hipMalloc(&d, 8) && !hipHostMalloc(&h, 8, 0) && !hipStreamCreateWithFlags(&s, 0), "owner");
-        check(d == hc.dev && h == hc.host && s == hc.stream, "the same addresses");
+        check(!hipMalloc(&d, 8) && !hipHostMalloc(&h, 8, 0), "owner");
+        check(d == hc.dev && h == hc.host, "the same addresses");
         hc.need(1000);
         usable(hc, 1000);
-        check(live.size() == 6 && hc.dev != d && hc.host != h && hc.stream != s, "the owner keeps its own");
-        hipFree(d), hipHostFree(h), hipStreamDestroy(s);
+        check(live.size() == 4 && hc.dev != d && hc.host != h, "the owner keeps its own");
+        hipFree(d), hipHostFree(h);
 
-        for (int k = 0; k < 3; k++) {   // each allocation of a set fails: nothing is kept
+        for (int k = 0; k < 2; k++) {   // each allocation of a set fails: nothing is kept
             live.clear();
             fail_after = k;
             bool thrown = false;
