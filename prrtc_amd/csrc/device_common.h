@@ -147,6 +147,26 @@ __device__ inline void bind_scene(const float *packed, int cap_f4, float4 *lds, 
     obs.bind(h, lds);
 }
 
+// The items 0 .. n - 1 of a launch that workgroup blockIdx.x takes, by first,
+// end and stride.  Workgroups reach the XCDs round-robin (workgroup b runs on
+// XCD b % 8) and each XCD has its own L2, so each XCD's workgroups share one
+// contiguous range: what neighbouring items read (an edge list's lines, a
+// tree) comes into one L2 instead of all eight.
+struct XcdRange {
+    int first, end, stride;
+    __device__ __forceinline__ explicit XcdRange(int n) {
+        first = blockIdx.x;
+        end = n;
+        stride = gridDim.x;
+        if ((int)gridDim.x >= kXcds) {
+            const int x = blockIdx.x % kXcds;
+            first = (int)((long long)n * x / kXcds) + blockIdx.x / kXcds;
+            end = (int)((long long)n * (x + 1) / kXcds);
+            stride = ((int)gridDim.x - x + kXcds - 1) / kXcds;   // workgroups on this XCD
+        }
+    }
+};
+
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 
 // Obstacle table read.  LOCAL: the tables are known to be staged in LDS, so
